@@ -4,17 +4,20 @@
 //
 // Those kernels are serial K loops whose whole output tile lives in the
 // register file as loop-carried fragments, one block per SM (255 registers).
-// This file has two kernels instead:
-//   * gemm_dma_kernel (the production path, tile codes 1-10): A and B tiles go
-//     straight from global memory into an S-stage LDS ring with
+// The kernels here and in gemm_pipe.hip work tile by tile instead:
+//   * gemm_pipe_kernel (gemm_pipe.hip; tile codes 1 and 9): large tiles, the K
+//     loop software-pipelined across its barrier;
+//   * gemm_dma_kernel (tile codes 2-8, 10, 15; 1 for an implicit convolution):
+//     A and B tiles go straight from global memory into an S-stage LDS ring with
 //     global_load_lds_dwordx4, XOR-swizzled for conflict-free MFMA operand
 //     reads; v_mfma_f32_32x32x16_f16 on a grid of 64x64 wave tiles (32x96 on
 //     the 128x96 QKV tile); one or two K-groups; an LDS-staged epilogue
 //     (described at the kernel);
+//   * gemm_kn_rb_kernel (tile code 2 with a [K][N] B): B through registers;
 //   * gemm_kernel (tile codes 11-14): register-staged loads with rows padded
 //     to 72 halves, kept for a B operand given as [K][N], which it transposes
 //     in registers.
-// Both split K over extra workgroups when the output has too few tiles to
+// All split K over extra workgroups when the output has too few tiles to
 // fill 256 CUs (the graph-level split-K the reference names as its next
 // lever, README.md:170-175), writing f32 partials that a reduce kernel -- or
 // the LayerNorm that consumes them -- sums in split order (deterministic,
@@ -30,13 +33,14 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm_common.h"
+#include "gemm_pipe.h"
 #include "gemv_block.h"
 #include "kernels.h"
 
 namespace ck {
 namespace {
 
-constexpr int BK = 64;
 // LDS ring stages of the LDS-DMA kernel's two-K-group configurations, and
 // whether the f32 staging of both groups (8 regions of (BM/2) x (BN/2 + 8)
 // floats) fits in that ring.
@@ -45,28 +49,6 @@ constexpr int dma_stages_kg2(int BM, int BN) {
 }
 constexpr bool kg2_staging_fits(int BM, int BN, int S) { return 2 * 4 * (BM / 2) * (BN / 2 + 8) * 4 <= S * (BM + BN) * BK * 2; }
 constexpr int LDK = BK + 8;   // padded LDS row (halves)
-
-struct GemmParams {
-  const half_t* A;
-  const half_t* B;
-  void* C;
-  const float* bias;
-  float* ws;
-  half_t* vt;
-  long lda, ldb, ldc, vt_ld;
-  long sA, sB, sC, sBias;
-  int M, N, K, kps;   // kps: K per split
-  int split, batch, Mt, Nt;
-  int qk_cols;
-  int head_dim;       // EPI_QKV_FRAG
-  int vec;            // 1: shapes/alignment allow the LDS-staged 16-byte epilogue
-  const half_t* pos;  // EPI_EMBED
-  const float* ctx;   // EPI_EMBED
-  int cc_log2, ch, cw, cwo;   // implicit conv: log2(channels), input height/width, output width
-  const half_t* zero;         // implicit conv: 16 zero bytes
-  int c_nm;                   // the split-K reduce stores element (m, n) at C[n*ldc + m]
-  unsigned* pair;             // split 2, f32 output: ticket counters of the in-kernel finish (null: a reduce follows)
-};
 
 // Implicit 3x3 stride-2 pad-1 convolution: the A chunk (8 halves) of patch
 // row m, columns k .. k+7 (one tap, 8 channels: C >= 8) is input pixel
@@ -78,34 +60,6 @@ __device__ __forceinline__ const half_t* conv_a_src(const GemmParams& p, const h
   const int y = yb + dy, x = xb + tap - 3 * dy;
   const bool ok = tap < 9 && (unsigned)y < (unsigned)p.ch && (unsigned)x < (unsigned)p.cw;
   return ok ? img + (((long)y * p.cw + x) << p.cc_log2) + c : p.zero;
-}
-
-template <int EPI>
-__device__ __forceinline__ void epi_store(const GemmParams& p, void* C, const float* bias, int m, int n, float v) {
-  if (EPI == EPI_F32) {
-    if (bias) v += bias[n];
-    static_cast<float*>(C)[(long)m * p.ldc + n] = v;
-  } else if (EPI == EPI_EMBED) {
-    if (bias) v += bias[n];
-    static_cast<float*>(C)[(long)m * p.ldc + n] = v + ((float)p.pos[(long)m * p.ldc + n] + p.ctx[n]);
-  } else if (EPI == EPI_F32_RESID) {
-    if (bias) v += bias[n];
-    float* c = static_cast<float*>(C) + (long)m * p.ldc + n;
-    *c = *c + v;
-  } else {
-    if (bias) v += bias[n];
-    if (EPI == EPI_F16_BIAS_RELU) v = fmaxf(v, 0.f);
-    if (EPI == EPI_F16_BIAS_GELU) v = gelu_fast(v);
-    if (EPI == EPI_QKV_FRAG) {
-      return;   // unreachable: the host admits EPI_QKV_FRAG only with the staged epilogue
-    } else if (EPI == EPI_QKV && n >= p.qk_cols) {
-      p.vt[(long)(n - p.qk_cols) * p.vt_ld + m] = (half_t)v;
-    } else if (p.c_nm) {
-      static_cast<half_t*>(C)[(long)n * p.ldc + m] = (half_t)v;
-    } else {
-      static_cast<half_t*>(C)[(long)m * p.ldc + n] = (half_t)v;
-    }
-  }
 }
 
 // 8x8 transpose of f16 values held as 8 rows of 4 packed words.
@@ -372,9 +326,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_gemv_kernel(const GemmParam
 // ---------------------------------------------------------------------------
 
 // Issue one K-step's loads of this wave into LDS stage `st` (A rows then B rows).
-// ko: the K-step's offset in A (halves); bko: in B (ko for a [N][K] B, ko
-// rows of ldb for a [K][N] B).  BPOL: the B loads' cache policy (0, or 2 =
-// non-temporal, see gemm_dma_kernel).
+// ko, bko: the K-step's offsets in A and B (halves).  BPOL: the B loads' cache
+// policy (0, or 2 = non-temporal, see gemm_dma_kernel).
 template <int NIA, int NIB, int STAGE_A, int BPOL = 0>
 __device__ __forceinline__ void dma_issue(const half_t* const* asrc, const half_t* const* bsrc, half_t* st, int wave,
                                           int ko, long bko) {
@@ -385,228 +338,6 @@ __device__ __forceinline__ void dma_issue(const half_t* const* asrc, const half_
   for (int i = 0; i < NIB; ++i)
     __builtin_amdgcn_global_load_lds(bsrc[i] + bko, (lds_ptr_t)(st + STAGE_A + (wave * NIB + i) * 8 * BK), 16, 0,
                                      BPOL);
-}
-
-// Coalesced epilogue.  The MFMA accumulator layout gives a lane one column
-// and scattered rows, so direct stores are 2- or 4-byte pieces spread over
-// 32 rows per instruction (and, for the transposed V of the QKV epilogue,
-// over 32 V^T rows).  Instead each wave puts its finished (WM x WN) sub-tile
-// -- bias and activation applied, converted to the output type -- into a
-// private LDS region and writes it out as whole 16-byte row chunks.  V
-// columns are staged transposed ([n][m]), four consecutive rows of a lane
-// forming one 8-byte LDS write, so V^T rows leave contiguously as well.
-// Row pitches carry 16 bytes of padding so the two half-waves' staging
-// writes (rows r and r+4) fall in different banks.  Every staged output --
-// split-K partials, f32 outputs (plain, residual-add, embedding), row-major
-// f16 outputs and the QKV fragments, all read by the next kernel -- leaves
-// with the device-scope cache policy (store_sc1: -0.5%, -0.4% and -0.3% of
-// the 1B frame for the partials, the f16 outputs and the fragments against
-// non-temporal or default stores) wherever the region is addressable by a
-// 32-bit buffer offset (sc1_ok), and with non-temporal stores otherwise.
-// Requires (checked on the host, else the direct per-element stores run):
-// N % 8 == 0, ldc / batch stride / base of C and ws 16-byte compatible,
-// and for QKV qk_cols % BN == 0 (% 32 on the 128x96 tile), M % 8 == 0 and
-// vt_ld % 8 == 0.
-//
-// EPI_QKV_FRAG writes the attention kernel's MFMA operands directly, in
-// 16-byte chunks ordered so that one wave's fragment load is one contiguous
-// KB (16 lanes x 16 B per row of the fragment would otherwise touch 16
-// separate rows).  With T = M tokens, d = qk_cols / 2, hd = head_dim,
-// H = d / hd, chunk c of a fragment holds 8 halves for lane l = 16*g + r:
-//   Q, K (16x16x32 A/B operand: row r = token, 8 head dims from 8*g):
-//     C chunk (((w*H + h) * T/16 + t/16) * hd/32 + j/32) * 64 + 16*((j%32)/8) + t%16
-//     for token t, head dim j of head h; w = 0 for Q, 1 for K.
-//   V (B operand of P.V: column r = head dim, tokens 4g..4g+3 and
-//   16+4g..16+4g+3 of a 32-token block, the attention kernel's key order):
-//     vt chunk ((h * hd/16 + j/16) * T/32 + t/32) * 64 + 16*((t%16)/4) + j%16,
-//     element (t/16)*4 + t%4 of the chunk.
-// SWP (every epilogue but the QKV ones): the accumulators hold D^T (the MFMA
-// ran with its operands swapped), so element e of tile (i, j) is row
-// i*32 + lane%32, column j*32 + 8*(e/4) + 4*(lane/32) + e%4: a lane's four
-// consecutive e are four consecutive columns of one row, staged with one 8-
-// or 16-byte LDS write instead of four scalar ones; bcol[j][e] is the bias
-// of that column (bcol[j][0] of column j*32 + lane%32 otherwise).
-template <int WM, int WN, int FM, int FN, int EPI, bool SWP, int NBC>
-__device__ __forceinline__ void store_staged(const GemmParams& p, const float16_t (&acc)[FM][FN],
-                                             const float (&bcol)[FN][NBC], char* region, int mw, int nw, int sp,
-                                             int bz, int lane) {
-  const bool to_ws = p.split > 1 || EPI == EPI_PARTIALS;
-  if (to_ws || EPI == EPI_F32 || EPI == EPI_F32_RESID || EPI == EPI_EMBED) {
-    constexpr int PF = WN + 8;   // floats
-    float* st = reinterpret_cast<float*>(region);
-    if constexpr (SWP) {
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float4_t v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * k + e] + bcol[j][4 * k + e];
-            *reinterpret_cast<float4_t*>(st + (i * 32 + (lane & 31)) * PF + j * 32 + 8 * k + 4 * (lane >> 5)) = v;
-          }
-    } else {
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int c = j * 32 + (lane & 31);
-        const float bv = bcol[j][0];
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            st[(i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * PF + c] = acc[i][j][e] + bv;
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-    constexpr int CPR = WN / 4;   // 16-byte chunks per row
-    float* dst = to_ws ? p.ws + ((long)sp * p.batch + bz) * (long)p.M * p.N : static_cast<float*>(p.C) + bz * p.sC;
-    const long ld = to_ws ? p.N : p.ldc;
-    const long plane = to_ws ? 4L * p.M * p.N : 4L * ((long)(p.M - 1) * p.ldc + p.N);
-    const bool sc1 = sc1_ok(plane);
-    const __amdgpu_buffer_rsrc_t rs = sc1_rsrc(dst, sc1 ? plane : 0);
-#pragma unroll 4
-    for (int q = lane; q < WM * CPR; q += 64) {
-      const int r = q / CPR, c = (q % CPR) * 4;
-      const int m = mw + r, n = nw + c;
-      if (m >= p.M || n >= p.N) continue;
-      float4_t v = *reinterpret_cast<const float4_t*>(st + r * PF + c);
-      float4_t* g = reinterpret_cast<float4_t*>(dst + (long)m * ld + n);
-      if (!to_ws && EPI == EPI_F32_RESID) v += *g;
-      if (!to_ws && EPI == EPI_EMBED) {
-        const half4_t ps = *reinterpret_cast<const half4_t*>(p.pos + (long)m * p.ldc + n);
-        const float4_t cs = *reinterpret_cast<const float4_t*>(p.ctx + n);
-        v += float4_t{(float)ps[0] + cs[0], (float)ps[1] + cs[1], (float)ps[2] + cs[2], (float)ps[3] + cs[3]};
-      }
-      if (sc1) store_sc1(rs, ((long)m * ld + n) * 4, v);
-      else __builtin_nontemporal_store(v, g);
-    }
-    return;
-  }
-  half_t* st = reinterpret_cast<half_t*>(region);
-  if ((EPI == EPI_QKV || EPI == EPI_QKV_FRAG) && nw >= p.qk_cols) {
-    constexpr int PT = WM + 8;   // halves, transposed rows [n][m]
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int c = j * 32 + (lane & 31);
-      const float bv = bcol[j][0];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          half4_t h;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = (half_t)(acc[i][j][4 * g4 + e] + bv);
-          *reinterpret_cast<half4_t*>(st + c * PT + i * 32 + 8 * g4 + 4 * (lane >> 5)) = h;
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-    if (EPI == EPI_QKV_FRAG) {
-      // V fragment blocks: 16 features x 32 tokens = 64 lanes x 8 tokens, one
-      // contiguous KB per block (see the layout note at the epilogue modes)
-      // The wave's WN columns lie in one head (head_dim is a power of two >= WN,
-      // checked on the host), so the head and the first 16-feature block are
-      // wave-uniform and the chunk index is shifts and adds.
-      const int r = lane & 15, g = lane >> 4, hs = __builtin_ctz(p.head_dim);
-      const int f0 = nw - p.qk_cols, h = f0 >> hs, c0 = f0 & (p.head_dim - 1);
-      const long cbase = (long)(h << (hs - 4)) + (c0 >> 4);   // 16-feature block of the wave's first column
-      const int tpb = p.M >> 5;                                 // 32-token blocks
-#pragma unroll
-      for (int blk = 0; blk < (WN / 16) * (WM / 32); ++blk) {
-        const int cb = blk % (WN / 16), tb = blk / (WN / 16);
-        if (mw + tb * 32 >= p.M) continue;
-        // tokens 4g..4g+3 and 16+4g..16+4g+3 of the 32-token block: the key
-        // order in which the attention kernel's P.V A operand leaves its softmax
-        const int nl = cb * 16 + r, ml = tb * 32 + g * 4;
-        const long chunk = ((cbase + cb) * tpb + (mw >> 5) + tb) * 64 + g * 16 + r;
-        const half4_t lo = *reinterpret_cast<const half4_t*>(st + nl * PT + ml);
-        const half4_t hi = *reinterpret_cast<const half4_t*>(st + nl * PT + ml + 16);
-        store_sc1(sc1_rsrc(p.vt, 2L * p.M * (p.N - p.qk_cols)), chunk * 16,
-                  half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
-      }
-      return;
-    }
-    constexpr int CPR = WM / 8;
-#pragma unroll 4
-    for (int q = lane; q < WN * CPR; q += 64) {
-      const int r = q / CPR, c = (q % CPR) * 8;
-      const int n = nw + r, m = mw + c;
-      if (n >= p.N || m >= p.M) continue;
-      *reinterpret_cast<half8_t*>(p.vt + (long)(n - p.qk_cols) * p.vt_ld + m) =
-          *reinterpret_cast<const half8_t*>(st + r * PT + c);
-    }
-    return;
-  }
-  constexpr int PH = WN + 8;   // halves
-  if constexpr (SWP) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          half4_t hv;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float v = acc[i][j][4 * k + e] + bcol[j][4 * k + e];
-            if (EPI == EPI_F16_BIAS_RELU) v = fmaxf(v, 0.f);
-            if (EPI == EPI_F16_BIAS_GELU) v = gelu_fast(v);
-            hv[e] = (half_t)v;
-          }
-          *reinterpret_cast<half4_t*>(st + (i * 32 + (lane & 31)) * PH + j * 32 + 8 * k + 4 * (lane >> 5)) = hv;
-        }
-  } else {
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int c = j * 32 + (lane & 31);
-      const float bv = bcol[j][0];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float v = acc[i][j][e] + bv;
-          if (EPI == EPI_F16_BIAS_RELU) v = fmaxf(v, 0.f);
-          if (EPI == EPI_F16_BIAS_GELU) v = gelu_fast(v);
-          st[(i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * PH + c] = (half_t)v;
-        }
-    }
-  }
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("" ::: "memory");
-  if (EPI == EPI_QKV_FRAG) {
-    // Q / K fragment blocks: 16 tokens x 32 features = 64 lanes x 8 features
-    // Q or K, the head and the first 32-feature block are wave-uniform (the
-    // wave's WN columns lie in one head, as for V above).
-    const int r = lane & 15, g = lane >> 4, hs = __builtin_ctz(p.head_dim), dh = p.qk_cols >> 1;
-    const int which = nw >= dh, f0 = nw - which * dh, h = f0 >> hs, c0 = f0 & (p.head_dim - 1);
-    const long hbase = (long)(which * (dh >> hs) + h) * (p.M >> 4);   // 16-token blocks before this head
-    const int kpb = p.head_dim >> 5;                                  // 32-feature blocks per head
-#pragma unroll
-    for (int blk = 0; blk < (WM / 16) * (WN / 32); ++blk) {
-      const int tb = blk % (WM / 16), kb = blk / (WM / 16);
-      if (mw + tb * 16 >= p.M) continue;
-      const int ml = tb * 16 + r, nl = kb * 32 + g * 8;
-      const long chunk = ((hbase + (mw >> 4) + tb) * kpb + (c0 >> 5) + kb) * 64 + g * 16 + r;
-      store_sc1(sc1_rsrc(p.C, 2L * p.M * p.qk_cols), chunk * 16, *reinterpret_cast<const half8_t*>(st + ml * PH + nl));
-    }
-    return;
-  }
-  constexpr int CPR = WN / 8;
-  half_t* dst = static_cast<half_t*>(p.C) + bz * p.sC;
-  const long span = 2L * ((long)(p.M - 1) * p.ldc + p.N);   // bytes of this batch's output
-  const bool sc1 = sc1_ok(span);
-  const __amdgpu_buffer_rsrc_t rs = sc1_rsrc(dst, sc1 ? span : 0);
-#pragma unroll 4
-  for (int q = lane; q < WM * CPR; q += 64) {
-    const int r = q / CPR, c = (q % CPR) * 8;
-    const int m = mw + r, n = nw + c;
-    if (m >= p.M || n >= p.N) continue;
-    const half8_t v = *reinterpret_cast<const half8_t*>(st + r * PH + c);
-    if (sc1) store_sc1(rs, ((long)m * p.ldc + n) * 2, v);
-    else __builtin_nontemporal_store(v, reinterpret_cast<half8_t*>(dst + (long)m * p.ldc + n));
-  }
 }
 
 // The QKV fragment epilogue for waves whose columns may straddle a head or
@@ -701,12 +432,6 @@ __device__ __forceinline__ void dma_issue_range(const half_t* const* asrc, const
                                        BPOL);
 }
 
-// Swizzle of a [K][N] B stage (rows of 128 halves = 16 chunks of 16 bytes):
-// physical chunk = logical chunk ^ bt_swz(row).  The 64 lanes of one
-// transposed fragment read cover rows r0..r0+3 and r0+8..r0+11 (r0 a multiple
-// of 4) x 4 chunks; the swizzle sends them to 16 distinct chunks, two lanes'
-// 8 bytes per chunk, the fewest passes 512 bytes take.
-__device__ __forceinline__ int bt_swz(int row) { return ((row & 3) << 2) | ((row >> 3) & 1); }
 
 // Split-K in pairs (split 2, f32 output, p.pair set; the staged two-group
 // epilogue): the two waves that computed the same rows of a sub-tile over
@@ -830,26 +555,15 @@ __device__ __forceinline__ void store_staged_kg2(const GemmParams& p, const floa
 // KG=2 puts 8 waves on a CU for one output tile (twice the loads in flight)
 // without a global split-K reduce; the groups' accumulators are summed
 // through LDS at the end (group 0 + group 1, fixed order).  A group's waves
-// form an (NWG/2) x 2 grid over the tile: NWG = 8 with a 256-row tile gives
-// every wave the same 64x64 sub-tile as NWG = 4 with 128 rows, while the CU
-// holds two waves per SIMD and each byte it loads feeds twice the MFMAs
-// along M.
-// BT: B is [K][N] (N contiguous, config 1's layout).  Its stage holds
-// B[k][n0 .. n0+127] rows (each DMA instruction fills 4 rows x 256 bytes),
-// and the MFMA B fragments come out of LDS transposed by
-// ds_read_b64_tr_b16: within a 16-lane group, source lane 4a+b reads 4
-// halves (n 4b..4b+3) of row a, and lane j receives element j%4 of source
-// lanes 4e + j/4, e = 0..3, i.e. rows 0..3 of column j.  Two such reads give
-// a lane the 8 consecutive k of its column.  Only 128x128 tiles with the f32
-// epilogue take this form.
+// form an (NWG/2) x 2 grid over the tile.
 // CV: A is an implicit convolution (conv_a_src): the A chunk addresses are
 // recomputed for every K-step instead of advancing by the step.
 // WCOL: waves across the tile's columns.  2 (every tile but one): a group's
 // waves form an (NWG/2) x 2 grid.  1: the 128x96 QKV tile, one wave per 32
 // rows over all 96 columns (store_qkv_frag_blocks).
-template <int BM, int BN, int S, int KG, int EPI, int NWG = 4, bool BT = false, bool CV = false, int WCOL = 2>
+template <int BM, int BN, int S, int KG, int EPI, int NWG = 4, bool CV = false, int WCOL = 2>
 __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParams p) {
-  static_assert(WCOL == 2 || (WCOL == 1 && EPI == EPI_QKV_FRAG && KG == 1 && !BT && !CV),
+  static_assert(WCOL == 2 || (WCOL == 1 && EPI == EPI_QKV_FRAG && KG == 1 && !CV),
                 "one wave column: the QKV fragment epilogue on one K-group only");
   constexpr int STAGE_A = BM * BK, STAGE_B = BN * BK, STAGE = STAGE_A + STAGE_B;   // halves
   static_assert(S % KG == 0 && S / KG >= 2, "each K-group owns at least two ring stages");
@@ -858,11 +572,7 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
   // The B (weight) stream of the tiles with 128 or more rows -- the 1B model's
   // block GEMMs, 8-34 MB of weights each -- is loaded non-temporal: -1.3% of
   // the 1B frame.  Smaller tiles serve GEMMs whose few MB of weights the other
-  // workgroups reuse from the caches (the 39M model: +2.4% with it).  The
-  // [K][N] B of config 1 streams non-temporal too: 32.1 -> 31.4 us.  (What
-  // still separates that kernel from the [N][K] one is texture-data time --
-  // TD busy 12.3 M against 8.8 M cycles for the same L2 requests -- not LDS
-  // bank conflicts, of which it has fewer.)
+  // workgroups reuse from the caches (the 39M model: +2.4% with it).
   constexpr int BPOL = BM >= 128 ? 2 : 0;
   __shared__ __attribute__((aligned(1024))) half_t lds[S * STAGE];
   constexpr int WM = BM / (NWG / WCOL), WN = BN / WCOL;
@@ -913,17 +623,10 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
   };
 #pragma unroll
   for (int i = 0; i < NIB; ++i) {
-    if (BT) {   // instruction i: stage rows (k) 4*(w4*NIB+i) .. +3, lane -> row +lane/16, physical chunk lane%16
-      const int r = (w4 * NIB + i) * 4 + (lane >> 4);
-      const int q = (lane & 15) ^ bt_swz(r);
-      bsrc[i] = p.B + bz * p.sB + (long)(kbeg + r) * p.ldb + n0 + q * 8;
-    } else {
-      const int r = (w4 * NIB + i) * 8 + (lane >> 3);
-      const int q = (lane & 7) ^ ((r >> 1) & 7);
-      bsrc[i] = p.B + bz * p.sB + (long)min(n0 + r, p.N - 1) * p.ldb + kbeg + q * 8;
-    }
+    const int r = (w4 * NIB + i) * 8 + (lane >> 3);
+    const int q = (lane & 7) ^ ((r >> 1) & 7);
+    bsrc[i] = p.B + bz * p.sB + (long)min(n0 + r, p.N - 1) * p.ldb + kbeg + q * 8;
   }
-  static_assert(!BT || (BN == 128 && EPI == EPI_F32), "[K][N] B: 128-wide N tiles and the f32 epilogue only");
   float16_t acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -934,13 +637,11 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
   // first vmcnt wait)
   // the epilogues of the tiles with two or more 32x32 products per wave run
   // the MFMA with swapped operands (accumulators = D^T; see store_staged),
-  // except the QKV ones and the [K][N] B path, whose transposed B reads
-  // measured slower in the other operand slot (config 1: 33.2 against
-  // 32.3 us).  On the 64x64 tiles (one product per wave) the 16 bias values
+  // except the QKV ones.  On the 64x64 tiles (one product per wave) the 16 bias values
   // per lane cost more than the staging writes save (39M frame 0.1870 ->
   // 0.1907 ms); the 1B model's O-projection (two per wave) gains (1B frame
   // 2.047 -> 2.036 ms).
-  constexpr bool SWP = EPI != EPI_QKV && EPI != EPI_QKV_FRAG && !BT && FM * FN >= 2;
+  constexpr bool SWP = EPI != EPI_QKV && EPI != EPI_QKV_FRAG && FM * FN >= 2;
   constexpr int NBC = SWP ? 16 : 1;
   float bcol[FN][NBC];
   {
@@ -958,7 +659,7 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
 #pragma unroll
   for (int t = 0; t < P; ++t)
     if (t < nkg) {
-      const long bko = BT ? (long)(KG * t + grp) * BK * p.ldb : (long)(KG * t + grp) * BK;
+      const long bko = (long)(KG * t + grp) * BK;
       if (CV) {
         const half_t* acv[NIA];
         conv_step(acv, KG * t + grp);
@@ -974,23 +675,6 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
 #pragma unroll
   for (int j = 0; j < FN; ++j) boff[j] = (wn * WN + j * 32 + (lane & 31)) * BK;
   const int rsw = (lane >> 1) & 7;   // ((row >> 1) & 7) of every fragment row this lane reads
-  // [K][N] B: lane (g = lane/16, a = (lane/4)%4, b = lane%4) of a transposed
-  // read of fragment j, k-half h (k = 8*(g/2) + 4h .. +3 of a 16-k slice,
-  // columns 16*(g%2) .. +15 of the fragment) reads row 8*(g/2) + 4h + a of the
-  // slice, halves 4b..4b+3 of the fragment's 16-column block; the row's
-  // swizzle does not depend on the slice (slices are 16 rows).
-  int btoff[FN][2];
-  if (BT) {
-    const int g = lane >> 4, a = (lane >> 2) & 3, b = lane & 3;
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 8 * (g >> 1) + 4 * h + a;
-        const int col = wn * WN + j * 32 + 16 * (g & 1) + 4 * b;
-        btoff[j][h] = row * BN + (((col >> 3) ^ bt_swz(row)) << 3) + (col & 7);
-      }
-  }
 
   for (int t = 0; t < nkg; ++t) {
     const int ahead = min(P - 1, nkg - 1 - t);   // this group's later steps already in flight
@@ -1007,7 +691,7 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
     const bool refill = t + P < nkg;
     half_t* const rst = lds + ((KG * (t + P) + grp) % S) * STAGE;
     const int rko = (KG * (t + P) + grp) * BK;
-    const long rbko = BT ? (long)rko * p.ldb : (long)rko;
+    const long rbko = rko;
     const half_t* acv[NIA];
     if (CV && refill) conv_step(acv, KG * (t + P) + grp);
     const half_t* const* ra = CV ? acv : asrc;
@@ -1026,18 +710,7 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
 #pragma unroll
       for (int i = 0; i < FM; ++i) af[kk][i] = *reinterpret_cast<const half8_t*>(sa + aoff[i] + ch);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        if (BT) {
-          typedef short s16x4_t __attribute__((ext_vector_type(4)));
-          typedef __attribute__((address_space(3))) s16x4_t* lds_s4_t;
-          const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t)(sb + kk * 16 * BN + btoff[j][0]));
-          const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t)(sb + kk * 16 * BN + btoff[j][1]));
-          const half4_t hl = __builtin_bit_cast(half4_t, lo), hh = __builtin_bit_cast(half4_t, hi);
-          bf[kk][j] = half8_t{hl[0], hl[1], hl[2], hl[3], hh[0], hh[1], hh[2], hh[3]};
-        } else {
-          bf[kk][j] = *reinterpret_cast<const half8_t*>(sb + boff[j] + ch);
-        }
-      }
+      for (int j = 0; j < FN; ++j) bf[kk][j] = *reinterpret_cast<const half8_t*>(sb + boff[j] + ch);
     };
     read_slice(0);
     read_slice(1);
@@ -1157,9 +830,7 @@ __global__ __launch_bounds__(64 * NWG * KG) void gemm_dma_kernel(const GemmParam
 // rather than the NT kernel's (n >> 1) & 7, and the upper half-wave writes
 // its columns in the order j ^ 1: both the fragment reads (16 consecutive
 // rows per pass) and the dword writes (64 lanes = 8 n-octets x 8 k-pairs)
-// then touch every bank at most once (a CPU replay checks both).  The transposing LDS reads of the
-// direct [K][N] path spend texture-data cycles (TD busy twice that of the
-// [N][K] kernel for the same L2 requests); this path does not.
+// then touch every bank at most once (a CPU replay checks both).
 // Per group step t (group step u = global step 2u + group):
 //   top:   wait for A(t) and B(t+1) (everything issued before step t-1), barrier
 //   then:  B(t+1) registers -> its LDS stage (read at step t-2, retired by
@@ -1436,15 +1107,15 @@ void launch_dma_tile_cv(const GemmParams& p, bool kg2, hipStream_t s) {
   constexpr int stage_bytes = (BM + BN) * BK * 2;
   constexpr int S1 = (5 * stage_bytes <= 163840) ? 5 : 4;
   constexpr int S2 = dma_stages_kg2(BM, BN);
-  if (kg2) CK_LAUNCH((gemm_dma_kernel<BM, BN, S2, 2, EPI, 4, false, true>), dim3(grid), dim3(512), 0, s, p);
-  else CK_LAUNCH((gemm_dma_kernel<BM, BN, S1, 1, EPI, 4, false, true>), dim3(grid), dim3(256), 0, s, p);
+  if (kg2) CK_LAUNCH((gemm_dma_kernel<BM, BN, S2, 2, EPI, 4, true>), dim3(grid), dim3(512), 0, s, p);
+  else CK_LAUNCH((gemm_dma_kernel<BM, BN, S1, 1, EPI, 4, true>), dim3(grid), dim3(256), 0, s, p);
   CK_LAUNCHED("gemm_dma_conv");
 }
 
 template <int EPI>
 void launch_epi_cv(int tile, const GemmParams& p, hipStream_t s) {
   if (tile == 15) {   // 32x64, two waves (short M: the conv stem's later layers)
-    CK_LAUNCH((gemm_dma_kernel<32, 64, 5, 1, EPI, 2, false, true>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(128),
+    CK_LAUNCH((gemm_dma_kernel<32, 64, 5, 1, EPI, 2, true>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(128),
               0, s, p);
     CK_LAUNCHED("gemm_dma_conv");
     return;
@@ -1459,25 +1130,6 @@ void launch_epi_cv(int tile, const GemmParams& p, hipStream_t s) {
   }
 }
 
-// LDS-DMA tiles for a [K][N] B (f32 output): 128x128 with two K-groups (tile
-// 1) or one, and 256x128 with 8 waves in one K-group (tile 9, 3-stage ring).
-void launch_dma_bt(const GemmParams& p, int tile, bool kg2, hipStream_t s) {
-  const int grid = p.Mt * p.Nt * p.split * p.batch;
-  if (tile == 9) CK_LAUNCH((gemm_dma_kernel<256, 128, 3, 1, EPI_F32, 8, true>), dim3(grid), dim3(512), 0, s, p);
-  else if (tile == 2) CK_LAUNCH(gemm_kn_rb_kernel, dim3(grid), dim3(512), 0, s, p);
-  else if (kg2) CK_LAUNCH((gemm_dma_kernel<128, 128, 4, 2, EPI_F32, 4, true>), dim3(grid), dim3(512), 0, s, p);
-  else CK_LAUNCH((gemm_dma_kernel<128, 128, 5, 1, EPI_F32, 4, true>), dim3(grid), dim3(256), 0, s, p);
-  CK_LAUNCHED("gemm_dma_bt");
-}
-
-// 256x128 tile: 8 waves of 64x64, one K-group, 3-stage ring (3 x 48 KB).
-template <int EPI>
-void launch_dma_tile8(const GemmParams& p, hipStream_t s) {
-  const int grid = p.Mt * p.Nt * p.split * p.batch;
-  CK_LAUNCH((gemm_dma_kernel<256, 128, 3, 1, EPI, 8>), dim3(grid), dim3(512), 0, s, p);
-  CK_LAUNCHED("gemm_dma");
-}
-
 template <int BM, int BN, bool BKN, int EPI>
 void launch_tile(const GemmParams& p, hipStream_t s) {
   const int grid = p.Mt * p.Nt * p.split * p.batch;
@@ -1486,10 +1138,11 @@ void launch_tile(const GemmParams& p, hipStream_t s) {
 }
 
 // tile codes (BM x BN): 1 128x128, 2 128x64, 3 64x128, 4 64x64.
-//   1-4: LDS-DMA kernel with two K-groups (8 waves) when K per split is a
-//        multiple of 128, else one group;  5-8: LDS-DMA, one group (a [K][N]
-//        B is first transposed into the workspace);
-//   9: 256x128 on the LDS-DMA kernel with 8 waves in one K-group;
+//   1, 9 (256x128): the pipelined kernel (gemm_pipe.hip), [N][K] or
+//        [K][N] B (implicit conv with tile 1: the LDS-DMA kernel);
+//   2-4: LDS-DMA kernel with two K-groups (8 waves) when K per split is a
+//        multiple of 128, else one group;  5-8: LDS-DMA, one group, 5 128x128
+//        (a [K][N] B is first transposed into the workspace);
 //   10: 128x96, one wave column (the QKV fragment epilogue only);
 //   11-14: register-staged kernel (a [K][N] B is transposed in registers);
 //   15: 32x64 on the LDS-DMA kernel with two waves ([N][K] B; implicit conv too).
@@ -1498,7 +1151,7 @@ void launch_epi(int tile, const GemmParams& p, hipStream_t s) {
   const int c = tile % 10;
   if (tile == 10) {   // 128x96, one wave column, 5-stage ring (5 x 28 KB): the QKV fragment epilogue only
     if constexpr (!BKN && EPI == EPI_QKV_FRAG) {
-      CK_LAUNCH((gemm_dma_kernel<128, 96, 5, 1, EPI, 4, false, false, 1>), dim3(p.Mt * p.Nt), dim3(256), 0, s, p);
+      CK_LAUNCH((gemm_dma_kernel<128, 96, 5, 1, EPI, 4, false, 1>), dim3(p.Mt * p.Nt), dim3(256), 0, s, p);
       CK_LAUNCHED("gemm_dma");
       return;
     }
@@ -1512,14 +1165,13 @@ void launch_epi(int tile, const GemmParams& p, hipStream_t s) {
     }
     throw Error("gemm: tile 15 (32x64) takes B as [N][K] only");
   }
-  if (!BKN && tile == 9) {
-    launch_dma_tile8<EPI>(p, s);
-    return;
-  }
   if (!BKN && tile < 10) {
     const bool kg2 = c <= 4 && p.kps % (2 * BK) == 0;
     switch (c > 4 ? c - 4 : c) {
-      case 1: launch_dma_tile<128, 128, EPI>(p, kg2, s); break;
+      case 1:
+        CK_LAUNCH((gemm_dma_kernel<128, 128, 5, 1, EPI>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(256), 0, s, p);
+        CK_LAUNCHED("gemm_dma");
+        break;
       case 2: launch_dma_tile<128, 64, EPI>(p, kg2, s); break;
       case 3: launch_dma_tile<64, 128, EPI>(p, kg2, s); break;
       default: launch_dma_tile<64, 64, EPI>(p, kg2, s); break;
@@ -1574,16 +1226,33 @@ void launch_reduce(const GemmParams& p, hipStream_t s, const GemvRider* rider = 
   CK_LAUNCHED("splitk_reduce_gemv");
 }
 
-// A [K][N] B on the two-K-group 128x128 LDS-DMA tile is streamed into LDS as
-// it lies and read transposed (no transpose pass, no workspace for it).
-// (A and B are required to be 16-byte aligned for every launch.)
+// The split-K reduce of an epilogue (EPI_PARTIALS leaves its partials to the
+// LayerNorm that consumes them).
+void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s) {
+  switch (epi) {
+    case EPI_F32: launch_reduce<EPI_F32>(p, s); break;
+    case EPI_F16_BIAS: launch_reduce<EPI_F16_BIAS>(p, s); break;
+    case EPI_F16_BIAS_RELU: launch_reduce<EPI_F16_BIAS_RELU>(p, s); break;
+    case EPI_F16_BIAS_GELU: launch_reduce<EPI_F16_BIAS_GELU>(p, s); break;
+    case EPI_F32_RESID: launch_reduce<EPI_F32_RESID>(p, s); break;
+    case EPI_EMBED: launch_reduce<EPI_EMBED>(p, s); break;
+    case EPI_QKV: launch_reduce<EPI_QKV>(p, s); break;
+    default: break;
+  }
+}
+
+// The tiles of the pipelined kernel (gemm_pipe.hip): 1 (128x128) and 9
+// (256x128), for everything but the implicit convolution.
+bool tile_pipe(const GemmDesc& d) { return (d.tile == 1 || d.tile == 9) && d.conv_c == 0; }
+
+// Tiles that take a [K][N] B as it lies (no transpose pass, no workspace for
+// it): the pipelined ones read it transposed out of LDS, tile 2 brings it in
+// through registers.
 bool bt_direct(const GemmDesc& d) {
   if (!d.b_kn) return false;
-  if (d.tile == 2)   // B through registers: whole 3-step phases of two K-groups
+  if (d.tile == 2)   // whole 3-step phases of two K-groups
     return d.N % 64 == 0 && (d.K / d.split) % (6 * BK) == 0;
-  if (d.N % 128 != 0) return false;
-  if (d.tile == 1) return (d.K / d.split) % (2 * BK) == 0;
-  return d.tile == 9;   // 256x128, 8 waves in one K-group
+  return tile_pipe(d);
 }
 
 // Ticket counters of the in-kernel split-2 finish (pair_finish): a static
@@ -1635,6 +1304,28 @@ unsigned* pair_slot(hipStream_t s) {
   return g_pair_base[dev] + (size_t)slot * kPairTickets;
 }
 
+// Of the pipelined tiles, the one whose waves of 256 workgroups take least
+// time: a 64-wide K-step of a CU's tile and its fixed part (first loads,
+// epilogue), fitted to 2048x4096 at K = 256 and 2048 (two waves of 128x128
+// 16.7 and 42.4 us, one of 256x128 13.2 and 36.2 us; 4096x4096x4096: 150 and
+// 126 us).  One wave of 128x128 tiles is never slower than fewer, larger ones
+// (512x8192x2048: 22 against 28 us).
+int large_tile(const GemmDesc& d) {
+  struct Cost { int tile, bm, bn; float step, fixed; };
+  constexpr Cost costs[] = {{1, 128, 128, 0.46f, 4.f}, {9, 256, 128, 0.82f, 5.f}};
+  int best = 1;
+  float best_us = 0.f;
+  for (const Cost& c : costs) {
+    const long tiles = (long)ceil_div(d.M, c.bm) * ceil_div(d.N, c.bn) * d.batch;
+    const float us = (float)ceil_div(tiles, 256) * ((float)(d.K / BK) * c.step + c.fixed);
+    if (best_us == 0.f || us < best_us) {
+      best = c.tile;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 int tile_base(int tile) { const int c = tile % 10; return c > 4 ? c - 4 : c; }
 bool tile_dma(int tile) { return tile <= 10 || tile == 15; }
 int tile_bm(int tile) {
@@ -1670,8 +1361,11 @@ size_t gemm_plan(GemmDesc& d) {
     const long t = (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch;
     if (t < 64) bm = bn = 64;
     d.tile = bm == 128 ? (bn == 128 ? 1 : 2) : (bn == 128 ? 3 : 4);
+    if (d.tile == 1 && t > 256 && d.split <= 1) d.tile = large_tile(d);
   }
   CK_REQUIRE((d.tile >= 1 && d.tile <= 15), "gemm: unknown tile code");
+  // the QKV epilogues run on the LDS-DMA kernel's 128x128 tile
+  if ((d.epi == EPI_QKV || d.epi == EPI_QKV_FRAG) && (d.tile == 1 || d.tile == 9)) d.tile = 5;
   CK_REQUIRE(d.tile != 15 || !d.b_kn, "gemm: tile 15 (32x64) takes B as [N][K]");
   CK_REQUIRE(d.tile != 10 || (d.epi == EPI_QKV_FRAG && !d.b_kn && d.conv_c == 0),
              "gemm: tile 10 (128x96) serves the QKV fragment epilogue only");
@@ -1771,7 +1465,7 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
     p.vec = v ? 1 : 0;
   }
   // Split 2 with an f32 output on a kernel with the two-group staged
-  // epilogue (the [K][N] register-B tile 2; [N][K] LDS-DMA tiles 1-4 with
+  // epilogue (the [K][N] register-B tile 2; [N][K] LDS-DMA tiles 2-4 with
   // two K-groups whose staging fits the ring) finishes in the kernel
   // (pair_finish) instead of a reduce launch.  Its partial planes must be
   // addressable by 32-bit buffer offsets (device-scope stores and loads).
@@ -1779,7 +1473,7 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
   {
     const int bm = tile_bm(d.tile), bn = tile_bn(d.tile);
     const bool staged = d.b_kn ? (d.tile == 2 && bt_direct(d))
-                               : (d.tile >= 1 && d.tile <= 4 && p.kps % (2 * BK) == 0 &&
+                               : (d.tile >= 2 && d.tile <= 4 && p.kps % (2 * BK) == 0 &&
                                   kg2_staging_fits(bm, bn, dma_stages_kg2(bm, bn)));
     const long tickets = (long)d.batch * p.Mt * p.Nt * 4 * 2;
     if (staged && d.split == 2 && d.epi == EPI_F32 && p.vec && !conv && 4L * d.M * d.N < (1L << 31) &&
@@ -1813,12 +1507,14 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
     if (d.split > 1) launch_reduce<EPI_F32>(p, s);
     return;
   }
-  if (bt_direct(d)) {
-    // the [K][N] B straight into LDS, fragments read transposed (no transpose
-    // pass).  Only with two K-groups: on one (tile 5) the doubled fragment
-    // reads cost more than the transpose pass saves (config 1: 44.6 against
-    // 33.2 us; two K-groups 32.6 against 34.9 us).
-    launch_dma_bt(p, d.tile, true, s);
+  if (tile_pipe(d)) {
+    launch_gemm_pipe(tile_bm(d.tile), tile_bn(d.tile), d.b_kn, d.epi, p, s);
+    if (d.split > 1) launch_reduce_epi(d.epi, p, s);
+    return;
+  }
+  if (bt_direct(d)) {   // tile 2
+    CK_LAUNCH(gemm_kn_rb_kernel, dim3(p.Mt * p.Nt * p.split * p.batch), dim3(512), 0, s, p);
+    CK_LAUNCHED("gemm_kn_rb");
     if (d.split > 1 && !p.pair) launch_reduce<EPI_F32>(p, s);
     return;
   }
@@ -1837,17 +1533,18 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
     return;
   }
   switch (d.epi) {
-    case EPI_F32: launch_epi<false, EPI_F32>(d.tile, p, s); if (d.split > 1 && !p.pair) launch_reduce<EPI_F32>(p, s); break;
-    case EPI_F16_BIAS: launch_epi<false, EPI_F16_BIAS>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_F16_BIAS>(p, s); break;
-    case EPI_F16_BIAS_RELU: launch_epi<false, EPI_F16_BIAS_RELU>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_F16_BIAS_RELU>(p, s); break;
-    case EPI_F16_BIAS_GELU: launch_epi<false, EPI_F16_BIAS_GELU>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_F16_BIAS_GELU>(p, s); break;
-    case EPI_F32_RESID: launch_epi<false, EPI_F32_RESID>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_F32_RESID>(p, s); break;
-    case EPI_EMBED: launch_epi<false, EPI_EMBED>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_EMBED>(p, s); break;
-    case EPI_QKV: launch_epi<false, EPI_QKV>(d.tile, p, s); if (d.split > 1) launch_reduce<EPI_QKV>(p, s); break;
+    case EPI_F32: launch_epi<false, EPI_F32>(d.tile, p, s); break;
+    case EPI_F16_BIAS: launch_epi<false, EPI_F16_BIAS>(d.tile, p, s); break;
+    case EPI_F16_BIAS_RELU: launch_epi<false, EPI_F16_BIAS_RELU>(d.tile, p, s); break;
+    case EPI_F16_BIAS_GELU: launch_epi<false, EPI_F16_BIAS_GELU>(d.tile, p, s); break;
+    case EPI_F32_RESID: launch_epi<false, EPI_F32_RESID>(d.tile, p, s); break;
+    case EPI_EMBED: launch_epi<false, EPI_EMBED>(d.tile, p, s); break;
+    case EPI_QKV: launch_epi<false, EPI_QKV>(d.tile, p, s); break;
     case EPI_PARTIALS: launch_epi<false, EPI_PARTIALS>(d.tile, p, s); break;
     case EPI_QKV_FRAG: launch_epi<false, EPI_QKV_FRAG>(d.tile, p, s); break;
     default: throw Error("gemm: unknown epilogue");
   }
+  if (d.split > 1 && !p.pair) launch_reduce_epi(d.epi, p, s);
 }
 
 }  // namespace ck

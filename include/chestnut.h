@@ -203,12 +203,12 @@ int ck_gemv(const void* W, const float* x, const float* bias, float* y, int rows
 
 /* C f32 [M][N] = A f16 [M][K] (lda) * B, B f16 either [K][N] (b_kn = 1, ldb)
  * or [N][K] (b_kn = 0, ldb); optional bias f32 [N].  K % 64 == 0.
- * tile: 0 auto, 1 128x128, 2 128x64, 3 64x128, 4 64x64 (5-8: the same tiles
- * with one K-group; 9: 256x128 with 8 waves; 11, 13: the register-staged
- * kernel; 10, 128x96, serves only the frame plan's QKV epilogue; 15: 32x64
- * with two waves, B as [N][K]); split_k: 0 auto.
+ * tile: 0 auto, 1 128x128, 2 128x64, 3 64x128, 4 64x64, 9 256x128
+ * (5-8: tiles 1-4 on the LDS-DMA kernel with one K-group; 11, 13: the
+ * register-staged kernel; 10, 128x96, serves only the frame plan's QKV
+ * epilogue; 15: 32x64 with two waves, B as [N][K]); split_k: 0 auto.
  * workspace: split_k * M * N floats when split_k > 1, plus, for a [K][N] B
- * on tiles 1-8, N * K halves for B transposed to [N][K] (query with
+ * on tiles 2-8, N * K halves for B transposed to [N][K] (query with
  * ck_gemm_workspace, which also resolves auto tile/split).
  * split_k = 2 on tile 2 ([K][N] B) or on tiles 2-4 ([N][K] B, K per split a
  * multiple of 128) finishes inside the GEMM launch (no reduce launch): the

@@ -1,5 +1,5 @@
-"""CPU replay of the [K][N]-B LDS-DMA layout of gemm.hip (gemm_dma_kernel with
-BT): the DMA addressing and row swizzle that fill a 64x128 stage, the per-lane
+"""CPU replay of the [K][N]-B LDS-DMA layout of gemm_pipe.hip (128-column
+tiles, BT): the DMA addressing and row swizzle that fill a 64x128 stage, the per-lane
 addresses of the transposed fragment reads, and the ds_read_b64_tr_b16 lane
 permutation (measured on gfx950 with an in-bounds probe: within a 16-lane
 group, result lane j element e = source lane 4e + j/4 element j%4) must give

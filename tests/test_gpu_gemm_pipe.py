@@ -1,0 +1,86 @@
+"""The pipelined GEMM tiles (1: 128x128, 9: 256x128) against the
+oracle where they can go wrong: one K-step up to more than the ring holds,
+ragged M and N around a tile edge, M-tile counts that do not fill a group of
+four, split K, outputs the 16-byte stores do not fit, every epilogue, B as
+[N][K] and [K][N].  Bounds: the f32 summation error of tests/test_gpu_kernels.py."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import kernels as OK
+from test_gpu_kernels import _gemm_check, dev, host
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -24
+
+
+@pytest.mark.parametrize('tile', [1, 9])
+@pytest.mark.parametrize('kn', [False, True])
+@pytest.mark.parametrize('M,N,Kd,split', [
+    (1, 8, 64, 1),            # one row, one 16-byte column chunk, one K-step
+    (257, 264, 128, 1),       # one past the 256 edge
+    (255, 120, 192, 1),       # one short of it
+    (129, 136, 256, 1), (300, 520, 320, 1), (130, 128, 448, 1),   # around the 3- and 4-stage rings
+    (1290, 392, 128, 1),      # 11 and 6 M-tiles: last group of four not full
+    (300, 520, 1024, 4), (128, 256, 384, 3)])
+def test_pipe_tiles_tails(gpu, tile, kn, M, N, Kd, split):
+    from chestnut import kernels as K
+    print(f'[gemm] pipe tile {tile} kn={kn} {M}x{N}x{Kd} split {split}', flush=True)
+    rng = np.random.default_rng(M + N + Kd + tile)
+    A = rng.standard_normal((M, Kd)).astype(np.float16)
+    B = rng.standard_normal((Kd, N) if kn else (N, Kd)).astype(np.float16)
+    b = rng.standard_normal(N).astype(np.float32)
+    C = host(K.gemm(dev(gpu, A), dev(gpu, B), b_kn=kn, bias=dev(gpu, b), tile=tile, split_k=split))
+    _gemm_check(C - b, A, B, transB=not kn, depth=Kd // 16 + 40)
+
+
+@pytest.mark.parametrize('tile', [1, 9])
+@pytest.mark.parametrize('kn,N,ldc', [(False, 201, 201), (False, 200, 203), (True, 200, 203)])
+@pytest.mark.parametrize('split', [1, 2])
+def test_pipe_tiles_without_16_byte_stores(gpu, tile, kn, N, ldc, split):
+    """N odd, or a row pitch that is no multiple of 16 bytes: stored per
+    element, and nothing outside [M][N] written."""
+    from chestnut import _lib
+    torch = gpu
+    M, Kd = 150, 256
+    rng = np.random.default_rng(N + ldc)
+    A = rng.standard_normal((M, Kd)).astype(np.float16)
+    B = rng.standard_normal((Kd, N) if kn else (N, Kd)).astype(np.float16)
+    Ad, Bd = dev(torch, A), dev(torch, B)
+    C = torch.full((M, ldc), 7.0, device='cuda')
+    ws = torch.empty(split * M * N, device='cuda')
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.call('ck_gemm', p(Ad), p(Bd), p(C), None, M, N, Kd, Kd, N if kn else Kd, ldc, 1 if kn else 0, tile, split,
+              p(ws), ws.numel() * 4, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    got = host(C)
+    _gemm_check(got[:, :N], A, B, transB=not kn)
+    assert (got[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize('tile', [1, 9])
+@pytest.mark.parametrize('M,N,split', [(200, 264, 1), (200, 260, 1), (130, 264, 2)])
+@pytest.mark.parametrize('epi', [1, 2, 3, 4])
+def test_pipe_tiles_epilogues(gpu, tile, M, N, split, epi):
+    from chestnut import kernels as K
+    torch = gpu
+    rng = np.random.default_rng(epi + N)
+    Kd = 256
+    A = (rng.standard_normal((M, Kd)) / 8).astype(np.float16)
+    W = (rng.standard_normal((N, Kd)) / 8).astype(np.float16)
+    b = rng.standard_normal(N).astype(np.float32)
+    acc = OK.gemm(A, W, transB=True) + b
+    if epi == 4:
+        C0 = rng.standard_normal((M, N)).astype(np.float32)
+        out = dev(torch, C0.copy())
+        K.gemm_epi(dev(torch, A), dev(torch, W), dev(torch, b), 4, out, tile=tile, split_k=split)
+        scale = np.abs(A.astype(np.float64)) @ np.abs(W.astype(np.float64)).T + np.abs(b) + np.abs(C0)
+        assert np.all(np.abs(host(out) - (C0 + acc)) <= (Kd // 16 + 40) * U * scale)
+        return
+    out = torch.empty(M, N, dtype=torch.float16, device='cuda')
+    K.gemm_epi(dev(torch, A), dev(torch, W), dev(torch, b), epi, out, tile=tile, split_k=split)
+    ref = {1: lambda v: v, 2: lambda v: np.maximum(v, 0), 3: OK.gelu}[epi](acc)
+    ref = ref.astype(np.float32).astype(np.float16).astype(np.float64)
+    # one f16 rounding of an f32 value within reassociation noise: at most one ulp apart
+    ulp = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
+    assert np.all(np.abs(host(out).astype(np.float64) - ref) <= ulp + 1e-7)
