@@ -52,8 +52,16 @@ constexpr int att_waves(int nkt) { return nkt <= 4 ? 2 * nkt : nkt; }
 
 // FRAG: qk / vt hold the operands in MFMA fragment order (written by the QKV
 // GEMM's fragment epilogue): every fragment load of a wave is one contiguous
-// KB.  Otherwise the row layouts: qk [T][2d], vt [d][T].  All of a wave's
-// loads (Q, its K, its V) are issued at entry, before any MFMA.
+// KB.  Otherwise the row layouts: qk [T][2d], vt [d][T].  There the two 16-key
+// tiles of a 32-key block take the keys 8q..8q+3 and 8q+4..8q+7 (q = 0..3) of
+// the block as their rows, so that the softmax leaves lane (g, r) the keys
+// 8g..8g+7: one 16-byte piece of a V^T row (in key order it is two 8-byte
+// pieces, twice the load instructions at half the bytes each; per launch, 16
+// heads of 128 at 512 tokens 16.1 -> 12.9 us, 12 at 384 12.7 -> 10.4, 8 heads of
+// 64 at 512 9.1 -> 7.4, at 256 5.7 -> 4.8).  Loading whole 128-byte lines and
+// exchanging halves between lanes, or spreading a head over the XCDs, measured
+// no faster (12.8 and 13.6 us).  All of a wave's loads (Q, its K, its V) are
+// issued at entry, before any MFMA.
 // QT: 16-query tiles per workgroup (2: 32 queries; 1: 16, twice the
 // workgroups for short sequences that would leave most CUs idle).
 // OTW > 0: the output projection rides along.  The workgroup's normalised
@@ -109,35 +117,45 @@ __global__ __launch_bounds__(64 * att_waves(NKT)) void attention_kernel(const ha
 
   // ---- all loads up front ----
   half8_t qf[QT][KS], kf[KT][KS], vb[KB][CT];
+  if constexpr (FRAG) {
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      kf[kt][ks] = *reinterpret_cast<const half8_t*>(
-          FRAG ? qk + ((((long)(n_heads + h) * (T / 16) + kw0 / 16 + kt) * KS + ks) * 64 + lane) * 8
-               : qk + (long)(kw0 + kt * 16 + r16) * ldq + d + h * HD + ks * 32 + g * 8);
+      for (int ks = 0; ks < KS; ++ks)
+        kf[kt][ks] = *reinterpret_cast<const half8_t*>(
+            qk + ((((long)(n_heads + h) * (T / 16) + kw0 / 16 + kt) * KS + ks) * 64 + lane) * 8);
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt)
+    for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[qt][ks] = *reinterpret_cast<const half8_t*>(
-          FRAG ? qk + ((((long)h * (T / 16) + q0 / 16 + qt) * KS + ks) * 64 + lane) * 8
-               : qk + (long)(q0 + qt * 16 + r16) * ldq + h * HD + ks * 32 + g * 8);
+      for (int ks = 0; ks < KS; ++ks)
+        qf[qt][ks] = *reinterpret_cast<const half8_t*>(
+            qk + ((((long)h * (T / 16) + q0 / 16 + qt) * KS + ks) * 64 + lane) * 8);
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      if (FRAG) {
+      for (int ct = 0; ct < CT; ++ct)
         vb[kb][ct] = *reinterpret_cast<const half8_t*>(
             vt + ((((long)h * (HD / 16) + ct) * (T / 32) + kw0 / 32 + kb) * 64 + lane) * 8);
-      } else {
-        // V^T row of feature ct*16 + r16: keys 4g..4g+3 and 16+4g..16+4g+3 of the block
-        const half_t* vr = vt + (long)(h * HD + ct * 16 + r16) * T + kw0 + kb * 32 + 4 * g;
-        const half4_t lo = *reinterpret_cast<const half4_t*>(vr);
-        const half4_t hi = *reinterpret_cast<const half4_t*>(vr + 16);
-        vb[kb][ct] = half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      }
+  } else {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      // tile row r is key (r / 4) * 8 + (kt % 2) * 4 + r % 4 of its 32-key block
+      const int key = kw0 + (kt >> 1) * 32 + (r16 >> 2) * 8 + (kt & 1) * 4 + (r16 & 3);
+      const half_t* kr = qk + (long)key * ldq + d + h * HD + g * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[kt][ks] = *reinterpret_cast<const half8_t*>(kr + ks * 32);
     }
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        qf[qt][ks] = *reinterpret_cast<const half8_t*>(qk + (long)(q0 + qt * 16 + r16) * ldq + h * HD + ks * 32 + g * 8);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        vb[kb][ct] = *reinterpret_cast<const half8_t*>(vt + (long)(h * HD + ct * 16 + r16) * T + kw0 + kb * 32 + 8 * g);
+  }
   // W_o fragments (MFMA A operand: row n = output feature, 8 k of head h's columns)
   half8_t wf[OTW > 0 ? OTW : 1][KSO];
   if constexpr (OTW > 0) {
