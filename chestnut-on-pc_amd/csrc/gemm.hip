@@ -5,8 +5,8 @@
 // Those kernels are serial K loops whose whole output tile lives in the
 // register file as loop-carried fragments, one block per SM (255 registers).
 // The kernels here and in gemm_pipe.hip work tile by tile instead:
-//   * gemm_pipe_kernel (gemm_pipe.hip; tile codes 1 and 9): large tiles, the K
-//     loop software-pipelined across its barrier;
+//   * gemm_pipe_kernel (gemm_pipe.hip; tile codes 1, 9 and 16): the K loop
+//     software-pipelined across its barrier, B as [N][K] or [K][N];
 //   * gemm_dma_kernel (tile codes 2-8, 10, 15; 1 for an implicit convolution):
 //     A and B tiles go straight from global memory into an S-stage LDS ring with
 //     global_load_lds_dwordx4, XOR-swizzled for conflict-free MFMA operand
@@ -27,6 +27,7 @@
 // MFMA 32x32x16 operand layout (lane l of 64): A row l%32, k = 8*(l/32)..+7;
 // B column l%32, same k; D element e of lane l is row 8*(e/4) + 4*(l/32) +
 // e%4, column l%32.  The layout is checked by the MFMA KAT (wmma.hip).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -1138,7 +1139,7 @@ void launch_tile(const GemmParams& p, hipStream_t s) {
 }
 
 // tile codes (BM x BN): 1 128x128, 2 128x64, 3 64x128, 4 64x64.
-//   1, 9 (256x128): the pipelined kernel (gemm_pipe.hip), [N][K] or
+//   1, 9 (256x128), 16 (64x64): the pipelined kernel (gemm_pipe.hip), [N][K] or
 //        [K][N] B (implicit conv with tile 1: the LDS-DMA kernel);
 //   2-4: LDS-DMA kernel with two K-groups (8 waves) when K per split is a
 //        multiple of 128, else one group;  5-8: LDS-DMA, one group, 5 128x128
@@ -1241,9 +1242,9 @@ void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s) {
   }
 }
 
-// The tiles of the pipelined kernel (gemm_pipe.hip): 1 (128x128) and 9
-// (256x128), for everything but the implicit convolution.
-bool tile_pipe(const GemmDesc& d) { return (d.tile == 1 || d.tile == 9) && d.conv_c == 0; }
+// The tiles of the pipelined kernel (gemm_pipe.hip): 1 (128x128), 9 (256x128)
+// and 16 (64x64), for everything but the implicit convolution.
+bool tile_pipe(const GemmDesc& d) { return (d.tile == 1 || d.tile == 9 || d.tile == 16) && d.conv_c == 0; }
 
 // Tiles that take a [K][N] B as it lies (no transpose pass, no workspace for
 // it): the pipelined ones read it transposed out of LDS, tile 2 brings it in
@@ -1304,34 +1305,55 @@ unsigned* pair_slot(hipStream_t s) {
   return g_pair_base[dev] + (size_t)slot * kPairTickets;
 }
 
-// Of the pipelined tiles, the one whose waves of 256 workgroups take least
-// time: a 64-wide K-step of a CU's tile and its fixed part (first loads,
-// epilogue), fitted to 2048x4096 at K = 256 and 2048 (two waves of 128x128
-// 16.7 and 42.4 us, one of 256x128 13.2 and 36.2 us; 4096x4096x4096: 150 and
-// 126 us).  One wave of 128x128 tiles is never slower than fewer, larger ones
-// (512x8192x2048: 22 against 28 us).
-int large_tile(const GemmDesc& d) {
-  struct Cost { int tile, bm, bn; float step, fixed; };
-  constexpr Cost costs[] = {{1, 128, 128, 0.46f, 4.f}, {9, 256, 128, 0.82f, 5.f}};
-  int best = 1;
-  float best_us = 0.f;
-  for (const Cost& c : costs) {
-    const long tiles = (long)ceil_div(d.M, c.bm) * ceil_div(d.N, c.bn) * d.batch;
-    const float us = (float)ceil_div(tiles, 256) * ((float)(d.K / BK) * c.step + c.fixed);
-    if (best_us == 0.f || us < best_us) {
-      best = c.tile;
-      best_us = us;
-    }
-  }
-  return best;
+// K split of the automatic choice: K of 16 steps or more takes the largest
+// split (<= 16) that divides the K-steps, leaves each split at least two of
+// them and keeps the grid within one wave of 256 CUs.  Shorter K is not split:
+// the partials and the reduce launch cost more than the extra workgroups gain
+// (measured on the conv stem: K = 576 runs 8.4 us unsplit, 10.0 us split in 3).
+int auto_split(long tiles, int ksteps) {
+  int s = 1;
+  if (ksteps >= 16)
+    for (int c = 2; c <= 16; ++c)
+      if (ksteps % c == 0 && ksteps / c >= 2 && tiles * c <= 256) s = c;
+  return s;
+}
+
+// Where 128x128 tiles number 64 or more: the tile whose estimated time is least
+// of 128x128 (with its automatic split), 256x128 and 64x64.  The estimates (us:
+// a fixed part, a part per 64-wide K-step of a CU's tile, per wave of 256
+// workgroups; two 64x64 workgroups share a CU) are fitted to replayed launches:
+//   128x128:  1000x1000x128 6.6, 128x8192x512 9.7, 1504x1504x1536 16.4,
+//             512x8192x2048 22, 2048x4096x2048 (two waves) 42.4
+//   256x128:  2048x4096x256 13.2, 2048x4096x2048 36.2
+//   64x64:    1000x1000x128 4.4, 128x8192x512 5.4, 1000x1000x1024 8.7 (128x128
+//             split in 4: 19.4), 1504x1504x1536 21.3, 700x3000x256 8.2
+//   reduce:   3 to 4 us and its bytes
+// 64x64 is tile 4 (two K-groups) for a few K-steps and for more of them tile 16
+// (pipelined, as many chains of roundings as the split it replaces).
+int tile_of_many(const GemmDesc& d) {
+  const int ks = d.K / BK;
+  const auto tiles = [&](int bm, int bn) { return (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch; };
+  const auto waves = [](long t) { return (float)((t + 255) / 256); };
+  const int s = d.split ? d.split : auto_split(tiles(128, 128), ks);
+  float best = 1.5f + waves(tiles(128, 128) * s) * (4.f + 0.46f * (float)(ks / s));
+  if (s > 1) best += 3.f + 0.1f * (float)s + (float)(s + 1) * (float)d.M * (float)d.N * 1e-6f;
+  int tile = 1;
+  const float t256 = 1.5f + waves(tiles(256, 128)) * (5.f + 0.82f * (float)ks);
+  if (s == 1 && t256 < best) best = t256, tile = 9;
+  const float w64 = (float)tiles(64, 64) / 256.f;
+  const float t64 = 3.f + 2.7f * std::max(0.f, w64 - 1.f) + 0.36f * (float)ks * std::max(1.f, w64);
+  if (t64 < best) tile = d.b_kn || ks >= 12 ? 16 : 4;
+  return tile;
 }
 
 int tile_base(int tile) { const int c = tile % 10; return c > 4 ? c - 4 : c; }
-bool tile_dma(int tile) { return tile <= 10 || tile == 15; }
+bool tile_dma(int tile) { return tile <= 10 || tile >= 15; }
 int tile_bm(int tile) {
+  if (tile == 16) return 64;
   return tile == 9 ? 256 : tile == 10 ? 128 : tile == 15 ? 32 : (tile_base(tile) == 1 || tile_base(tile) == 2) ? 128 : 64;
 }
 int tile_bn(int tile) {
+  if (tile == 16) return 64;
   return tile == 9 ? 128 : tile == 10 ? 96 : tile == 15 ? 64 : (tile_base(tile) == 1 || tile_base(tile) == 3) ? 128 : 64;
 }
 
@@ -1361,9 +1383,14 @@ size_t gemm_plan(GemmDesc& d) {
     const long t = (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch;
     if (t < 64) bm = bn = 64;
     d.tile = bm == 128 ? (bn == 128 ? 1 : 2) : (bn == 128 ? 3 : 4);
-    if (d.tile == 1 && t > 256 && d.split <= 1) d.tile = large_tile(d);
+    if (d.tile == 1 && d.split <= 1) d.tile = tile_of_many(d);
+    // a [K][N] B as it lies instead of a transpose pass over it (11x6272x832 14.5
+    // -> 7.8 us, 16x4096x4096 23.7 -> 13.1 us, 600x600x4096 21.8 -> 17.0 us)
+    if (d.b_kn && d.tile >= 2 && d.tile <= 4) d.tile = 16;
   }
-  CK_REQUIRE((d.tile >= 1 && d.tile <= 15), "gemm: unknown tile code");
+  CK_REQUIRE((d.tile >= 1 && d.tile <= 16), "gemm: unknown tile code");
+  CK_REQUIRE(d.tile != 16 || (d.epi != EPI_QKV && d.epi != EPI_QKV_FRAG && d.conv_c == 0),
+             "gemm: tile 16 (pipelined 64x64) takes neither the QKV epilogues nor an implicit conv");
   // the QKV epilogues run on the LDS-DMA kernel's 128x128 tile
   if ((d.epi == EPI_QKV || d.epi == EPI_QKV_FRAG) && (d.tile == 1 || d.tile == 9)) d.tile = 5;
   CK_REQUIRE(d.tile != 15 || !d.b_kn, "gemm: tile 15 (32x64) takes B as [N][K]");
@@ -1372,19 +1399,7 @@ size_t gemm_plan(GemmDesc& d) {
   if (d.b_kn && !tile_dma(d.tile))
     CK_REQUIRE(d.tile == 11 || d.tile == 13, "gemm: [K][N] B on the register-staged kernel needs a 128-wide N tile");
   const long tiles = (long)ceil_div(d.M, tile_bm(d.tile)) * ceil_div(d.N, tile_bn(d.tile)) * d.batch;
-  if (d.split == 0) {
-    // K of 16 steps or more: the largest split (<= 16) that divides the
-    // K-steps, leaves each split at least two of them and keeps the grid
-    // within one wave of 256 CUs.  Shorter K is not split: the partials and
-    // the reduce launch cost more than the extra workgroups gain (measured
-    // on the conv stem: K = 576 runs 8.4 us unsplit, 10.0 us split in 3).
-    const int ksteps = d.K / BK;
-    int s = 1;
-    if (ksteps >= 16)
-      for (int c = 2; c <= 16; ++c)
-        if (ksteps % c == 0 && ksteps / c >= 2 && tiles * c <= 256) s = c;
-    d.split = s;
-  }
+  if (d.split == 0) d.split = auto_split(tiles, d.K / BK);
   CK_REQUIRE(d.split >= 1 && d.K % (BK * d.split) == 0, "gemm: K must split into multiples of 64");
   // workspace: split-K partials, then (a [K][N] B on the LDS-DMA kernel) B transposed to [N][K] f16
   const size_t partials = (d.split > 1 || d.epi == EPI_PARTIALS) ? (size_t)d.split * d.batch * d.M * d.N : 0;

@@ -62,7 +62,7 @@ __device__ __forceinline__ void wait_steps(int later) {
 // loads of a stage in the first two slices after its barrier (else spread over
 // four); BT: B is [K][N].
 template <int BM, int BN, int S, int WGM, int WGN, bool FRONT, int EPI, bool BT>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmParams p) {
+__global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_kernel(const GemmParams p) {
   constexpr int NW = WGM * WGN;
   constexpr int STAGE_A = BM * BK * 2, STAGE = (BM + BN) * BK * 2;   // bytes
   constexpr int WM = BM / WGM, WN = BN / WGN, FM = WM / 32, FN = WN / 32, NM = FM * FN;
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
   for (int i = 0; i < NIB; ++i) {
     if (BT) {
       constexpr int CH = BN / 8;   // 16-byte chunks per stage row
-      const int c = (wave * NIB + i) * 64 + lane, r = c / CH, q = (c % CH) ^ bt_swz(r);
+      const int c = (wave * NIB + i) * 64 + lane, r = c / CH, q = (c % CH) ^ bt_swz<BN>(r);
       boff[i] = (long)r * p.ldb * 2 + min(n0 + q * 8, p.N - 8) * 2;
     } else {
       const int r = (wave * NIB + i) * 8 + (lane >> 3), q = (lane & 7) ^ ((r >> 1) & 7);
@@ -125,13 +125,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
                                        (lds_ptr_t)(st + STAGE_A + (wave * NIB + i - NIA) * 1024), 16, 0, 0);
   };
 
-  // two accumulators per product, for the even and the odd k-slices: each chain
-  // of roundings is half as long (relative error at K = 4096 2.9e-7, one chain 4.1e-7)
-  float16_t acc[2][FM][1][FN];
+  // NCH accumulators per product, each taking every NCH-th k-slice: a chain of
+  // roundings is that much shorter (relative error at K = 4096: one chain 4.1e-7,
+  // two 2.9e-7, eight 1.6e-7).  The 64x64 tile, whose products leave room for
+  // eight, then needs no split of K to be as exact as a split one was.
+  constexpr int NCH = NM == 1 ? 8 : 2;
+  float16_t acc[NCH][FM][1][FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int c = 0; c < NCH; ++c)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[0][i][0][j] = acc[1][i][0][j] = float16_t{};
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[c][i][0][j] = float16_t{};
 
   // the bias of the lane's epilogue columns: older than every DMA, so it has
   // landed by the first wait
@@ -172,7 +177,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
       for (int h = 0; h < 2; ++h) {
         const int row = 8 * (gq >> 1) + 4 * h + a;
         const int col = wn * WN + j * 32 + 16 * (gq & 1) + 4 * b;
-        btoff[j][h] = STAGE_A + (row * BN + (((col >> 3) ^ bt_swz(row)) << 3) + (col & 7)) * 2;
+        btoff[j][h] = STAGE_A + (row * BN + (((col >> 3) ^ bt_swz<BN>(row)) << 3) + (col & 7)) * 2;
       }
   }
   half8_t fa[2][FM], fb[2][FN];
@@ -191,19 +196,29 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
   // LDS-DMA load in flight has landed, as it cannot tell the stages apart.
   auto read_bt = [&](auto BUF, auto KK, unsigned so) {
     constexpr int bu = decltype(BUF)::value, kk = decltype(KK)::value;
-    static_assert(!BT || FN == 2, "transposed reads are written for two column fragments");
+    static_assert(!BT || FN <= 2, "transposed reads are written for one or two column fragments");
     u32x2_t v0, v1, v2, v3;
-    asm volatile(
-        "ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
-        "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
-        "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
-        "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
-        : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "v"(btoff[FN - 1][0] + so), "v"(btoff[FN - 1][1] + so),
-          "n"(kk * 16 * BN * 2));
-    fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
-    fb[bu][FN - 1] = __builtin_bit_cast(half8_t, u32x4_t{v2[0], v2[1], v3[0], v3[1]});
+    if constexpr (FN == 1) {
+      asm volatile(
+          "ds_read_b64_tr_b16 %0, %2 offset:%4\n\t"
+          "ds_read_b64_tr_b16 %1, %3 offset:%4\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(v0), "=&v"(v1)
+          : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "n"(kk * 16 * BN * 2));
+      fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
+    } else {
+      asm volatile(
+          "ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
+          "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
+          "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
+          "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
+          : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "v"(btoff[FN - 1][0] + so), "v"(btoff[FN - 1][1] + so),
+            "n"(kk * 16 * BN * 2));
+      fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
+      fb[bu][FN - 1] = __builtin_bit_cast(half8_t, u32x4_t{v2[0], v2[1], v3[0], v3[1]});
+    }
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -213,8 +228,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
   // One k-slice: the MFMAs of the fragments in buffer KK & 1, the reads of the
   // next slice (slice RK of the stage at `rso`) and NI / 4 refill loads placed
   // between them.
-  auto slice = [&](auto KK, auto RK, bool reads, unsigned rso, bool refill, lwr_t rst, gptr_t ra, gptr_t rb, auto DLO, auto DHI) {
-    constexpr int cur = decltype(KK)::value & 1;
+  auto slice = [&](auto PAR, auto KK, auto RK, bool reads, unsigned rso, bool refill, lwr_t rst, gptr_t ra, gptr_t rb, auto DLO, auto DHI) {
+    constexpr int cur = decltype(KK)::value & 1, ch = (4 * decltype(PAR)::value + decltype(KK)::value) % NCH;
     using NX = std::integral_constant<int, 1 - cur>;
     constexpr int dlo = decltype(DLO)::value, ND = decltype(DHI)::value - dlo;
     constexpr int RPM = (NR + NM - 1) / NM;   // reads per MFMA slot
@@ -222,7 +237,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
     for (int m = 0; m < NM; ++m) {
       const int i = m / FN, j = m % FN;
       // operands swapped: the accumulators hold D^T (see store_staged)
-      acc[cur][i][0][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[cur][j], fa[cur][i], acc[cur][i][0][j], 0, 0, 0);
+      acc[ch][i][0][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[cur][j], fa[cur][i], acc[ch][i][0][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (reads) {
 #pragma unroll
@@ -256,13 +271,13 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
   using D2 = std::integral_constant<int, E0>;
   using D3 = std::integral_constant<int, E1>;
   using D4 = std::integral_constant<int, NI>;
-  auto step = [&](auto MAIN, int t) {
+  auto step = [&](auto MAIN, auto PAR, int t) {
     constexpr bool main = decltype(MAIN)::value;
     const bool refp = main || (t >= 1 && t - 1 + S < nk), ref = main || t + S < nk, more = main || t + 1 < nk;
     const unsigned son = so + STAGE == S * STAGE ? 0u : so + STAGE;
-    slice(I0{}, I1{}, true, so, refp, lw + sop, ab, bb, D1{}, D2{});
-    slice(I1{}, I2{}, true, so, refp, lw + sop, ab, bb, D2{}, D3{});
-    slice(I2{}, I3{}, true, so, refp, lw + sop, ab, bb, D3{}, D4{});
+    slice(PAR, I0{}, I1{}, true, so, refp, lw + sop, ab, bb, D1{}, D2{});
+    slice(PAR, I1{}, I2{}, true, so, refp, lw + sop, ab, bb, D2{}, D3{});
+    slice(PAR, I2{}, I3{}, true, so, refp, lw + sop, ab, bb, D3{}, D4{});
     if (refp) {
       ab += astep;
       bb += bstep;
@@ -272,15 +287,38 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
       else wait_steps<S - 2, NI>(min(S - 2, nk - 2 - t));
       lds_barrier();
     }
-    slice(I3{}, I0{}, more, son, ref, lw + so, ab, bb, D0{}, D1{});
+    slice(PAR, I3{}, I0{}, more, son, ref, lw + so, ab, bb, D0{}, D1{});
     sop = so;
     so = son;
   };
-  step(std::false_type{}, 0);
+  using F = std::false_type;
+  using T = std::true_type;
   int t = 1;
-  for (; t + S < nk; ++t) step(std::true_type{}, t);
-  for (; t < nk; ++t) step(std::false_type{}, t);
+  step(F{}, I0{}, 0);
+  if constexpr (NCH <= 4) {
+    for (; t + S < nk; ++t) step(T{}, I0{}, t);
+    for (; t < nk; ++t) step(F{}, I0{}, t);
+  } else {   // odd steps take the second four accumulators
+    for (; t + 1 + S < nk; t += 2) {
+      step(T{}, I1{}, t);
+      step(T{}, I0{}, t + 1);
+    }
+    for (; t < nk; t += 2) {
+      step(F{}, I1{}, t);
+      if (t + 1 < nk) step(F{}, I0{}, t + 1);
+    }
+  }
 
+  // the chains' sum of product (i, j), by halves
+  auto chain_sum = [&](int i, int j) {
+    // (keeps the sums of later products behind this one's stores: all at once
+    // they do not fit the registers of the larger tiles)
+    if constexpr (NM > 1) asm volatile("" : "+a"(acc[1][i][0][j])::"memory");
+#pragma unroll
+    for (int w = 1; w < NCH; w *= 2)
+#pragma unroll
+      for (int c = 0; c + w < NCH; c += 2 * w) acc[c][i][0][j] += acc[c + w][i][0][j];
+  };
   if (!p.vec) {   // shapes or addresses the 16-byte stores do not fit
     const bool to_ws = p.split > 1 || EPI == EPI_PARTIALS;
     float* ws = p.ws + ((long)sp * p.batch + bz) * (long)p.M * p.N;
@@ -291,16 +329,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j) {
+        chain_sum(i, j);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int m = m0 + wm * WM + i * 32 + (lane & 31);
           const int n = n0 + wn * WN + j * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
           if (m >= p.M || n >= p.N) continue;
-          const float v = acc[0][i][0][j][e] + acc[1][i][0][j][e];
+          const float v = acc[0][i][0][j][e];
           if (to_ws) ws[(long)m * p.N + n] = v;
           else epi_store<EPI>(p, C, bias, m, n, v);
         }
+      }
     return;
   }
   // ---- staged epilogue: 32 rows of the wave's sub-tile at a time through LDS,
@@ -310,11 +350,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_pipe_kernel(const GemmPar
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      // (keeps the sums of later rows behind this one's stores: all at once they do not fit the registers)
-      asm volatile("" : "+a"(acc[1][i][0][j]));
-      acc[0][i][0][j] += acc[1][i][0][j];
-    }
+    for (int j = 0; j < FN; ++j) chain_sum(i, j);
     store_staged<32, WN, 1, FN, EPI, true, 16>(p, acc[0][i], bcol, lds + wave * REGION, m0 + wm * WM + i * 32, n0 + wn * WN,
                                                sp, bz, lane);
     __builtin_amdgcn_wave_barrier();
@@ -341,6 +377,7 @@ template <int EPI>
 void launch_e(int bm, int bn, bool b_kn, const GemmParams& p, hipStream_t s) {
   if (bm == 256 && bn == 128) launch_t<256, 128, 3, 2, 2, true, EPI>(b_kn, p, s);
   else if (bm == 128 && bn == 128) launch_t<128, 128, 4, 2, 2, false, EPI>(b_kn, p, s);
+  else if (bm == 64 && bn == 64) launch_t<64, 64, 4, 2, 2, false, EPI>(b_kn, p, s);
   else throw Error("gemm: no pipelined kernel for this tile");
 }
 

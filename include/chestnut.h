@@ -203,8 +203,8 @@ int ck_gemv(const void* W, const float* x, const float* bias, float* y, int rows
 
 /* C f32 [M][N] = A f16 [M][K] (lda) * B, B f16 either [K][N] (b_kn = 1, ldb)
  * or [N][K] (b_kn = 0, ldb); optional bias f32 [N].  K % 64 == 0.
- * tile: 0 auto, 1 128x128, 2 128x64, 3 64x128, 4 64x64, 9 256x128
- * (5-8: tiles 1-4 on the LDS-DMA kernel with one K-group; 11, 13: the
+ * tile: 0 auto, 1 128x128, 2 128x64, 3 64x128, 4 64x64, 9 256x128,
+ * 16 64x64 pipelined (5-8: tiles 1-4 on the LDS-DMA kernel with one K-group; 11, 13: the
  * register-staged kernel; 10, 128x96, serves only the frame plan's QKV
  * epilogue; 15: 32x64 with two waves, B as [N][K]); split_k: 0 auto.
  * workspace: split_k * M * N floats when split_k > 1, plus, for a [K][N] B
