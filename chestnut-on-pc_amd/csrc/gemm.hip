@@ -13,6 +13,7 @@
 //     reads; v_mfma_f32_32x32x16_f16 on a grid of 64x64 wave tiles (32x96 on
 //     the 128x96 QKV tile); one or two K-groups; an LDS-staged epilogue
 //     (described at the kernel);
+//   * gemm_small_kernel (gemm_small.hip; tile code 17): few tiles and a long K;
 //   * gemm_kn_rb_kernel (tile code 2 with a [K][N] B): B through registers;
 //   * gemm_kernel (tile codes 11-14): register-staged loads with rows padded
 //     to 72 halves, kept for a B operand given as [K][N], which it transposes
@@ -255,37 +256,7 @@ __device__ __forceinline__ void splitk_reduce_at(const GemmParams& p, long t) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += part[i][e];
   }
-  void* C = (EPI == EPI_F32 || EPI == EPI_F32_RESID || EPI == EPI_EMBED)
-                ? static_cast<void*>(static_cast<float*>(p.C) + bz * p.sC)
-                : static_cast<void*>(static_cast<half_t*>(p.C) + bz * p.sC);
-  const float* bias = p.bias ? p.bias + bz * p.sBias : nullptr;
-  // Row-major outputs take the thread's 4 values in one 16-byte (f32) or
-  // 8-byte (f16) store where the address allows: the same values as
-  // epi_store, a quarter of the store instructions.
-  if (v4 && (EPI == EPI_F32 || ((EPI == EPI_F16_BIAS || EPI == EPI_F16_BIAS_RELU || EPI == EPI_F16_BIAS_GELU) &&
-                                !p.c_nm))) {
-    float o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[e] = bias ? v[e] + bias[n + e] : v[e];
-      if (EPI == EPI_F16_BIAS_RELU) o[e] = fmaxf(o[e], 0.f);
-      if (EPI == EPI_F16_BIAS_GELU) o[e] = gelu_fast(o[e]);
-    }
-    if (EPI == EPI_F32) {
-      float* c = static_cast<float*>(C) + (long)m * p.ldc + n;
-      if ((reinterpret_cast<uintptr_t>(c) & 15) == 0) {
-        *reinterpret_cast<float4_t*>(c) = float4_t{o[0], o[1], o[2], o[3]};
-        return;
-      }
-    } else {
-      half_t* c = static_cast<half_t*>(C) + (long)m * p.ldc + n;
-      if ((reinterpret_cast<uintptr_t>(c) & 7) == 0) {
-        *reinterpret_cast<half4_t*>(c) = half4_t{(half_t)o[0], (half_t)o[1], (half_t)o[2], (half_t)o[3]};
-        return;
-      }
-    }
-  }
-  for (int e = 0; e < per; ++e) epi_store<EPI>(p, C, bias, m, n + e, v[e]);
+  store_reduced<EPI>(p, bz, m, n, v, per, v4);
 }
 
 template <int EPI>
@@ -1146,7 +1117,8 @@ void launch_tile(const GemmParams& p, hipStream_t s) {
 //        (a [K][N] B is first transposed into the workspace);
 //   10: 128x96, one wave column (the QKV fragment epilogue only);
 //   11-14: register-staged kernel (a [K][N] B is transposed in registers);
-//   15: 32x64 on the LDS-DMA kernel with two waves ([N][K] B; implicit conv too).
+//   15: 32x64 on the LDS-DMA kernel with two waves ([N][K] B; implicit conv too);
+//   17: 32x32, K over the four waves (gemm_small.hip; [N][K] B, no split).
 template <bool BKN, int EPI>
 void launch_epi(int tile, const GemmParams& p, hipStream_t s) {
   const int c = tile % 10;
@@ -1305,6 +1277,17 @@ unsigned* pair_slot(hipStream_t s) {
   return g_pair_base[dev] + (size_t)slot * kPairTickets;
 }
 
+int tile_base(int tile) { const int c = tile % 10; return c > 4 ? c - 4 : c; }
+bool tile_dma(int tile) { return tile <= 10 || tile >= 15; }
+int tile_bm(int tile) {
+  if (tile >= 16) return tile == 17 ? 32 : 64;
+  return tile == 9 ? 256 : tile == 10 ? 128 : tile == 15 ? 32 : (tile_base(tile) == 1 || tile_base(tile) == 2) ? 128 : 64;
+}
+int tile_bn(int tile) {
+  if (tile >= 16) return tile == 17 ? 32 : 64;
+  return tile == 9 ? 128 : tile == 10 ? 96 : tile == 15 ? 64 : (tile_base(tile) == 1 || tile_base(tile) == 3) ? 128 : 64;
+}
+
 // K split of the automatic choice: K of 16 steps or more takes the largest
 // split (<= 16) that divides the K-steps, leaves each split at least two of
 // them and keeps the grid within one wave of 256 CUs.  Shorter K is not split:
@@ -1346,15 +1329,23 @@ int tile_of_many(const GemmDesc& d) {
   return tile;
 }
 
-int tile_base(int tile) { const int c = tile % 10; return c > 4 ? c - 4 : c; }
-bool tile_dma(int tile) { return tile <= 10 || tile >= 15; }
-int tile_bm(int tile) {
-  if (tile == 16) return 64;
-  return tile == 9 ? 256 : tile == 10 ? 128 : tile == 15 ? 32 : (tile_base(tile) == 1 || tile_base(tile) == 2) ? 128 : 64;
-}
-int tile_bn(int tile) {
-  if (tile == 16) return 64;
-  return tile == 9 ? 128 : tile == 10 ? 96 : tile == 15 ? 64 : (tile_base(tile) == 1 || tile_base(tile) == 3) ? 128 : 64;
+// Where 128x128 tiles are fewer than 64, or M or N at most 64: whether 32x32
+// tiles with K over the waves (tile 17) beat the 64-wide tile with its automatic
+// split.  Estimates as above, fitted to replayed launches (us, tile 17 against
+// the other): 200x520x2048 5.9 / 7.9 (split 4), 16x4096x4096 8.5 / 12.2 (split 4),
+// 11x6272x832 4.7 / 7.3, 600x600x4096 14.1 / 15.8 (split 2), 256x2048x512 5.0 / 4.7,
+// 1x1024x8192 11.7 / 10.0 (split 16); a call of two launches takes 8 us of host
+// time at least.  Not where the split has more chains of roundings than the 16
+// that tile 17 sums an element in.
+bool small_tiles_win(const GemmDesc& d) {
+  const int ks = d.K / BK;
+  const auto tiles = [&](int bm, int bn) { return (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch; };
+  const int s = d.split ? d.split : auto_split(tiles(tile_bm(d.tile), tile_bn(d.tile)), ks);
+  if (s * (ks / s % 2 == 0 ? 2 : 1) > 16) return false;
+  const float w = (float)tiles(32, 32) / 256.f;
+  const float t17 = 2.8f + (float)ks * std::max(0.085f, 0.13f * w) + 0.8f * std::max(0.f, w - 1.f);
+  const float other = 3.f + 0.3f * (float)(ks / s) + (s > 1 ? 3.5f + 0.1f * (float)s : 0.f);
+  return t17 < other;
 }
 
 }  // namespace
@@ -1384,13 +1375,23 @@ size_t gemm_plan(GemmDesc& d) {
     if (t < 64) bm = bn = 64;
     d.tile = bm == 128 ? (bn == 128 ? 1 : 2) : (bn == 128 ? 3 : 4);
     if (d.tile == 1 && d.split <= 1) d.tile = tile_of_many(d);
+    if (!d.b_kn && d.tile >= 2 && d.tile <= 4 && d.split <= 1) {
+      // one 64-wide dimension and a K too short to split: 64x64 keeps twice the
+      // CUs busy (128x8192x512 on 64x128 7.6, on 64x64 5.5 us)
+      if (d.K / BK < 16) d.tile = 4;
+      if (small_tiles_win(d)) d.tile = 17;
+    }
     // a [K][N] B as it lies instead of a transpose pass over it (11x6272x832 14.5
     // -> 7.8 us, 16x4096x4096 23.7 -> 13.1 us, 600x600x4096 21.8 -> 17.0 us)
     if (d.b_kn && d.tile >= 2 && d.tile <= 4) d.tile = 16;
   }
-  CK_REQUIRE((d.tile >= 1 && d.tile <= 16), "gemm: unknown tile code");
+  CK_REQUIRE((d.tile >= 1 && d.tile <= 17), "gemm: unknown tile code");
   CK_REQUIRE(d.tile != 16 || (d.epi != EPI_QKV && d.epi != EPI_QKV_FRAG && d.conv_c == 0),
              "gemm: tile 16 (pipelined 64x64) takes neither the QKV epilogues nor an implicit conv");
+  CK_REQUIRE(d.tile != 17 || (!d.b_kn && d.split <= 1 && d.conv_c == 0 &&
+                              (d.epi == EPI_F32 || d.epi == EPI_F16_BIAS || d.epi == EPI_F16_BIAS_RELU ||
+                               d.epi == EPI_F16_BIAS_GELU || d.epi == EPI_F32_RESID)),
+             "gemm: tile 17 (32x32, K over the waves) takes B as [N][K], split 1 and the f32, f16 and residual epilogues");
   // the QKV epilogues run on the LDS-DMA kernel's 128x128 tile
   if ((d.epi == EPI_QKV || d.epi == EPI_QKV_FRAG) && (d.tile == 1 || d.tile == 9)) d.tile = 5;
   CK_REQUIRE(d.tile != 15 || !d.b_kn, "gemm: tile 15 (32x64) takes B as [N][K]");
@@ -1399,7 +1400,7 @@ size_t gemm_plan(GemmDesc& d) {
   if (d.b_kn && !tile_dma(d.tile))
     CK_REQUIRE(d.tile == 11 || d.tile == 13, "gemm: [K][N] B on the register-staged kernel needs a 128-wide N tile");
   const long tiles = (long)ceil_div(d.M, tile_bm(d.tile)) * ceil_div(d.N, tile_bn(d.tile)) * d.batch;
-  if (d.split == 0) d.split = auto_split(tiles, d.K / BK);
+  if (d.split == 0) d.split = d.tile == 17 ? 1 : auto_split(tiles, d.K / BK);
   CK_REQUIRE(d.split >= 1 && d.K % (BK * d.split) == 0, "gemm: K must split into multiples of 64");
   // workspace: split-K partials, then (a [K][N] B on the LDS-DMA kernel) B transposed to [N][K] f16
   const size_t partials = (d.split > 1 || d.epi == EPI_PARTIALS) ? (size_t)d.split * d.batch * d.M * d.N : 0;
@@ -1520,6 +1521,10 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
   if (d.b_kn && !tile_dma(d.tile)) {
     launch_epi<true, EPI_F32>(d.tile, p, s);
     if (d.split > 1) launch_reduce<EPI_F32>(p, s);
+    return;
+  }
+  if (d.tile == 17) {
+    launch_gemm_small(d.epi, p, s);
     return;
   }
   if (tile_pipe(d)) {

@@ -59,6 +59,52 @@ __device__ __forceinline__ void epi_store(const GemmParams& p, void* C, const fl
   }
 }
 
+// The epilogue of `per` summed values of row m, columns n.. (4 of them with v4):
+// row-major outputs take 4 values in one 16-byte (f32) or 8-byte (f16) store
+// where the address allows, the same values as epi_store.
+template <int EPI>
+__device__ __forceinline__ void store_reduced(const GemmParams& p, int bz, int m, int n, const float (&v)[4], int per,
+                                              bool v4) {
+  void* C = (EPI == EPI_F32 || EPI == EPI_F32_RESID || EPI == EPI_EMBED)
+                ? static_cast<void*>(static_cast<float*>(p.C) + bz * p.sC)
+                : static_cast<void*>(static_cast<half_t*>(p.C) + bz * p.sC);
+  const float* bias = p.bias ? p.bias + bz * p.sBias : nullptr;
+  if (v4 && (EPI == EPI_F32 || ((EPI == EPI_F16_BIAS || EPI == EPI_F16_BIAS_RELU || EPI == EPI_F16_BIAS_GELU) &&
+                                !p.c_nm))) {
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = bias ? v[e] + bias[n + e] : v[e];
+      if (EPI == EPI_F16_BIAS_RELU) o[e] = fmaxf(o[e], 0.f);
+      if (EPI == EPI_F16_BIAS_GELU) o[e] = gelu_fast(o[e]);
+    }
+    if (EPI == EPI_F32) {
+      float* c = static_cast<float*>(C) + (long)m * p.ldc + n;
+      if ((reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+        *reinterpret_cast<float4_t*>(c) = float4_t{o[0], o[1], o[2], o[3]};
+        return;
+      }
+    } else {
+      half_t* c = static_cast<half_t*>(C) + (long)m * p.ldc + n;
+      if ((reinterpret_cast<uintptr_t>(c) & 7) == 0) {
+        *reinterpret_cast<half4_t*>(c) = half4_t{(half_t)o[0], (half_t)o[1], (half_t)o[2], (half_t)o[3]};
+        return;
+      }
+    }
+  }
+  if (v4 && EPI == EPI_F32_RESID) {
+    float4_t* c = reinterpret_cast<float4_t*>(static_cast<float*>(C) + (long)m * p.ldc + n);
+    if ((reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+      float4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = bias ? v[e] + bias[n + e] : v[e];
+      *c = *c + o;
+      return;
+    }
+  }
+  for (int e = 0; e < per; ++e) epi_store<EPI>(p, C, bias, m, n + e, v[e]);
+}
+
 // Coalesced epilogue.  The MFMA accumulator layout gives a lane one column
 // and scattered rows, so direct stores are 2- or 4-byte pieces spread over
 // 32 rows per instruction (and, for the transposed V of the QKV epilogue,

@@ -62,7 +62,7 @@ __device__ __forceinline__ void wait_steps(int later) {
 // loads of a stage in the first two slices after its barrier (else spread over
 // four); BT: B is [K][N].
 template <int BM, int BN, int S, int WGM, int WGN, bool FRONT, int EPI, bool BT>
-__global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_kernel(const GemmParams p) {
+__global__ __launch_bounds__(64 * WGM * WGN, BM == 64 && S <= 4 ? 2 : 1) void gemm_pipe_kernel(const GemmParams p) {
   constexpr int NW = WGM * WGN;
   constexpr int STAGE_A = BM * BK * 2, STAGE = (BM + BN) * BK * 2;   // bytes
   constexpr int WM = BM / WGM, WN = BN / WGN, FM = WM / 32, FN = WN / 32, NM = FM * FN;
@@ -196,29 +196,19 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_ke
   // LDS-DMA load in flight has landed, as it cannot tell the stages apart.
   auto read_bt = [&](auto BUF, auto KK, unsigned so) {
     constexpr int bu = decltype(BUF)::value, kk = decltype(KK)::value;
-    static_assert(!BT || FN <= 2, "transposed reads are written for one or two column fragments");
+    static_assert(!BT || NM == 1 || FN == 2, "transposed reads are written for two column fragments");
     u32x2_t v0, v1, v2, v3;
-    if constexpr (FN == 1) {
-      asm volatile(
-          "ds_read_b64_tr_b16 %0, %2 offset:%4\n\t"
-          "ds_read_b64_tr_b16 %1, %3 offset:%4\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(v0), "=&v"(v1)
-          : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "n"(kk * 16 * BN * 2));
-      fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
-    } else {
-      asm volatile(
-          "ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
-          "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
-          "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
-          "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
-          : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "v"(btoff[FN - 1][0] + so), "v"(btoff[FN - 1][1] + so),
-            "n"(kk * 16 * BN * 2));
-      fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
-      fb[bu][FN - 1] = __builtin_bit_cast(half8_t, u32x4_t{v2[0], v2[1], v3[0], v3[1]});
-    }
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
+        "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
+        "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
+        "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
+        : "v"(btoff[0][0] + so), "v"(btoff[0][1] + so), "v"(btoff[FN - 1][0] + so), "v"(btoff[FN - 1][1] + so),
+          "n"(kk * 16 * BN * 2));
+    fb[bu][0] = __builtin_bit_cast(half8_t, u32x4_t{v0[0], v0[1], v1[0], v1[1]});
+    fb[bu][FN - 1] = __builtin_bit_cast(half8_t, u32x4_t{v2[0], v2[1], v3[0], v3[1]});
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -228,8 +218,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_ke
   // One k-slice: the MFMAs of the fragments in buffer KK & 1, the reads of the
   // next slice (slice RK of the stage at `rso`) and NI / 4 refill loads placed
   // between them.
-  auto slice = [&](auto PAR, auto KK, auto RK, bool reads, unsigned rso, bool refill, lwr_t rst, gptr_t ra, gptr_t rb, auto DLO, auto DHI) {
-    constexpr int cur = decltype(KK)::value & 1, ch = (4 * decltype(PAR)::value + decltype(KK)::value) % NCH;
+  auto slice = [&](auto KK, auto RK, bool reads, unsigned rso, bool refill, lwr_t rst, gptr_t ra, gptr_t rb, auto DLO, auto DHI) {
+    constexpr int cur = decltype(KK)::value & 1;
     using NX = std::integral_constant<int, 1 - cur>;
     constexpr int dlo = decltype(DLO)::value, ND = decltype(DHI)::value - dlo;
     constexpr int RPM = (NR + NM - 1) / NM;   // reads per MFMA slot
@@ -237,7 +227,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_ke
     for (int m = 0; m < NM; ++m) {
       const int i = m / FN, j = m % FN;
       // operands swapped: the accumulators hold D^T (see store_staged)
-      acc[ch][i][0][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[cur][j], fa[cur][i], acc[ch][i][0][j], 0, 0, 0);
+      acc[cur][i][0][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[cur][j], fa[cur][i], acc[cur][i][0][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (reads) {
 #pragma unroll
@@ -254,59 +244,130 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 ? 2 : 1) void gemm_pipe_ke
     }
   };
 
-  // stage offsets (bytes) of steps t-1, t, t+1
-  unsigned so = 0, sop = 0;
-  wait_steps<S - 1, NI>(min(S, nk) - 1);   // step 0's loads
-  lds_barrier();
-#pragma unroll
-  for (int r = 0; r < (BT ? FM : NR); ++r) read_one(I0{}, I0{}, r, 0u);
-  if (BT) read_bt(I0{}, I0{}, 0u);
-
-  // ab, bb point at the step whose refill is being issued: step t-1+S in slices 0..2 of step t
-  // (its first quarter went out in slice 3 of step t-1), step t+S in slice 3
-  // refill loads issued by the end of slices 3, 0 and 1 (slice 2 issues the rest)
-  constexpr int E3 = FRONT ? NI / 2 : NI / 4, E0 = FRONT ? NI : NI / 2, E1 = FRONT ? NI : NI * 3 / 4;
-  using D0 = std::integral_constant<int, 0>;
-  using D1 = std::integral_constant<int, E3>;
-  using D2 = std::integral_constant<int, E0>;
-  using D3 = std::integral_constant<int, E1>;
-  using D4 = std::integral_constant<int, NI>;
-  auto step = [&](auto MAIN, auto PAR, int t) {
-    constexpr bool main = decltype(MAIN)::value;
-    const bool refp = main || (t >= 1 && t - 1 + S < nk), ref = main || t + S < nk, more = main || t + 1 < nk;
-    const unsigned son = so + STAGE == S * STAGE ? 0u : so + STAGE;
-    slice(PAR, I0{}, I1{}, true, so, refp, lw + sop, ab, bb, D1{}, D2{});
-    slice(PAR, I1{}, I2{}, true, so, refp, lw + sop, ab, bb, D2{}, D3{});
-    slice(PAR, I2{}, I3{}, true, so, refp, lw + sop, ab, bb, D3{}, D4{});
-    if (refp) {
-      ab += astep;
-      bb += bstep;
-    }
-    if (more) {
-      if (main) wait_vm_lgkm0<(S - 2) * NI>();
-      else wait_steps<S - 2, NI>(min(S - 2, nk - 2 - t));
-      lds_barrier();
-    }
-    slice(PAR, I3{}, I0{}, more, son, ref, lw + so, ab, bb, D0{}, D1{});
-    sop = so;
-    so = son;
-  };
   using F = std::false_type;
   using T = std::true_type;
-  int t = 1;
-  step(F{}, I0{}, 0);
-  if constexpr (NCH <= 4) {
-    for (; t + S < nk; ++t) step(T{}, I0{}, t);
-    for (; t < nk; ++t) step(F{}, I0{}, t);
-  } else {   // odd steps take the second four accumulators
+  // stage offsets (bytes) of step t and, for the larger tiles, t - 1
+  unsigned so = 0;
+  wait_steps<S - 1, NI>(min(S, nk) - 1);   // step 0's loads
+  lds_barrier();
+  if constexpr (NM == 1) {
+    // One product per wave: a slice's MFMA covers a quarter of an LDS round trip,
+    // so the fragments of the whole next step are read while this step's MFMAs
+    // run, in registers of the other parity.
+    half8_t ga[2][KS], gb[2][KS];
+    auto read_a = [&](auto BUF, unsigned o) {
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+        ga[decltype(BUF)::value][kk] = *(const __attribute__((address_space(3))) half8_t*)(lr + ((arow + o) ^ (kk << 5)));
+    };
+    auto read_b = [&](auto BUF, unsigned o) {
+      constexpr int bu = decltype(BUF)::value;
+      if constexpr (BT) {
+        u32x2_t v[2 * KS];
+        asm volatile(   // see read_bt
+            "ds_read_b64_tr_b16 %0, %8\n\t"
+            "ds_read_b64_tr_b16 %1, %9\n\t"
+            "ds_read_b64_tr_b16 %2, %8 offset:%10\n\t"
+            "ds_read_b64_tr_b16 %3, %9 offset:%10\n\t"
+            "ds_read_b64_tr_b16 %4, %8 offset:%11\n\t"
+            "ds_read_b64_tr_b16 %5, %9 offset:%11\n\t"
+            "ds_read_b64_tr_b16 %6, %8 offset:%12\n\t"
+            "ds_read_b64_tr_b16 %7, %9 offset:%12\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+            : "v"(btoff[0][0] + o), "v"(btoff[0][1] + o), "n"(16 * BN * 2), "n"(32 * BN * 2), "n"(48 * BN * 2));
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk)
+          gb[bu][kk] = __builtin_bit_cast(half8_t, u32x4_t{v[2 * kk][0], v[2 * kk][1], v[2 * kk + 1][0], v[2 * kk + 1][1]});
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk)
+          gb[bu][kk] = *(const __attribute__((address_space(3))) half8_t*)(lr + ((brow + o) ^ (kk << 5)));
+      }
+    };
+    read_a(I0{}, 0u);
+    read_b(I0{}, 0u);
+    // ab, bb point at step t + S
+    auto step = [&](auto MAIN, auto PAR, int t) {
+      constexpr bool main = decltype(MAIN)::value;
+      constexpr int par = decltype(PAR)::value;
+      using NX = std::integral_constant<int, 1 - par>;
+      const bool ref = main || t + S < nk, more = main || t + 1 < nk;
+      const unsigned son = so + STAGE == S * STAGE ? 0u : so + STAGE;
+      if (more) {
+        // step t + 1 has landed, and this wave's reads of stage t have
+        if (main) wait_vm_lgkm0<(S - 2) * NI>();
+        else wait_steps<S - 2, NI>(min(S - 2, nk - 2 - t));
+        lds_barrier();
+        read_a(NX{}, son);
+        if (!BT) read_b(NX{}, son);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        acc[4 * par + kk][0][0][0] =
+            __builtin_amdgcn_mfma_f32_32x32x16_f16(gb[par][kk], ga[par][kk], acc[4 * par + kk][0][0][0], 0, 0, 0);
+        if (ref) {
+#pragma unroll
+          for (int i = kk * NI / KS; i < (kk + 1) * NI / KS; ++i) dma(i, ab, bb, lw + so);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (ref) {
+        ab += astep;
+        bb += bstep;
+      }
+      if (BT && more) read_b(NX{}, son);
+      so = son;
+    };
+    int t = 0;
     for (; t + 1 + S < nk; t += 2) {
-      step(T{}, I1{}, t);
-      step(T{}, I0{}, t + 1);
+      step(T{}, I0{}, t);
+      step(T{}, I1{}, t + 1);
     }
     for (; t < nk; t += 2) {
-      step(F{}, I1{}, t);
-      if (t + 1 < nk) step(F{}, I0{}, t + 1);
+      step(F{}, I0{}, t);
+      if (t + 1 < nk) step(F{}, I1{}, t + 1);
     }
+  } else {
+    unsigned sop = 0;
+#pragma unroll
+    for (int r = 0; r < (BT ? FM : NR); ++r) read_one(I0{}, I0{}, r, 0u);
+    if (BT) read_bt(I0{}, I0{}, 0u);
+
+    // ab, bb point at the step whose refill is being issued: step t-1+S in slices 0..2 of step t
+    // (its first quarter went out in slice 3 of step t-1), step t+S in slice 3
+    // refill loads issued by the end of slices 3, 0 and 1 (slice 2 issues the rest)
+    constexpr int E3 = FRONT ? NI / 2 : NI / 4, E0 = FRONT ? NI : NI / 2, E1 = FRONT ? NI : NI * 3 / 4;
+    using D0 = std::integral_constant<int, 0>;
+    using D1 = std::integral_constant<int, E3>;
+    using D2 = std::integral_constant<int, E0>;
+    using D3 = std::integral_constant<int, E1>;
+    using D4 = std::integral_constant<int, NI>;
+    auto step = [&](auto MAIN, int t) {
+      constexpr bool main = decltype(MAIN)::value;
+      const bool refp = main || (t >= 1 && t - 1 + S < nk), ref = main || t + S < nk, more = main || t + 1 < nk;
+      const unsigned son = so + STAGE == S * STAGE ? 0u : so + STAGE;
+      slice(I0{}, I1{}, true, so, refp, lw + sop, ab, bb, D1{}, D2{});
+      slice(I1{}, I2{}, true, so, refp, lw + sop, ab, bb, D2{}, D3{});
+      slice(I2{}, I3{}, true, so, refp, lw + sop, ab, bb, D3{}, D4{});
+      if (refp) {
+        ab += astep;
+        bb += bstep;
+      }
+      if (more) {
+        if (main) wait_vm_lgkm0<(S - 2) * NI>();
+        else wait_steps<S - 2, NI>(min(S - 2, nk - 2 - t));
+        lds_barrier();
+      }
+      slice(I3{}, I0{}, more, son, ref, lw + so, ab, bb, D0{}, D1{});
+      sop = so;
+      so = son;
+    };
+    int t = 1;
+    step(F{}, 0);
+    for (; t + S < nk; ++t) step(T{}, t);
+    for (; t < nk; ++t) step(F{}, t);
   }
 
   // the chains' sum of product (i, j), by halves
@@ -377,6 +438,7 @@ template <int EPI>
 void launch_e(int bm, int bn, bool b_kn, const GemmParams& p, hipStream_t s) {
   if (bm == 256 && bn == 128) launch_t<256, 128, 3, 2, 2, true, EPI>(b_kn, p, s);
   else if (bm == 128 && bn == 128) launch_t<128, 128, 4, 2, 2, false, EPI>(b_kn, p, s);
+  else if (bm == 64 && bn == 64 && p.Mt * p.Nt * p.split * p.batch <= 256) launch_t<64, 64, 8, 2, 2, false, EPI>(b_kn, p, s);
   else if (bm == 64 && bn == 64) launch_t<64, 64, 4, 2, 2, false, EPI>(b_kn, p, s);
   else throw Error("gemm: no pipelined kernel for this tile");
 }

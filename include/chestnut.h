@@ -206,7 +206,8 @@ int ck_gemv(const void* W, const float* x, const float* bias, float* y, int rows
  * tile: 0 auto, 1 128x128, 2 128x64, 3 64x128, 4 64x64, 9 256x128,
  * 16 64x64 pipelined (5-8: tiles 1-4 on the LDS-DMA kernel with one K-group; 11, 13: the
  * register-staged kernel; 10, 128x96, serves only the frame plan's QKV
- * epilogue; 15: 32x64 with two waves, B as [N][K]); split_k: 0 auto.
+ * epilogue; 15: 32x64 with two waves, B as [N][K]; 17: 32x32 with K over the
+ * waves, B as [N][K], split 1); split_k: 0 auto.
  * workspace: split_k * M * N floats when split_k > 1, plus, for a [K][N] B
  * on tiles 2-8, N * K halves for B transposed to [N][K] (query with
  * ck_gemm_workspace, which also resolves auto tile/split).

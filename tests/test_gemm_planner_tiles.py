@@ -29,6 +29,10 @@ def test_planner_takes_the_tile_with_the_cheapest_waves(kn, M, N, K, tile):
     (1000, 1000, 128, 1, 16, 1),
     (221, 4120, 64, 0, 4, 1),         # 66 of 128x128, 260 of 64x64
     (1504, 1504, 1536, 0, 1, 1),      # 144 of 128x128 for 24 K-steps
+    (200, 520, 2048, 0, 17, 1),       # few tiles, long K: 32x32 instead of a split in 4
+    (11, 6272, 832, 0, 17, 1), (16, 4096, 4096, 0, 17, 1), (64, 8192, 512, 0, 4, 1),
+    (256, 2048, 512, 0, 4, 1),        # 512 tiles of 32x32
+    (64, 512, 4096, 0, 4, 16), (40, 40, 8192, 0, 4, 16),   # splits with more chains of roundings
     (11, 6272, 832, 1, 16, 1),        # few rows: B read as it lies
     (16, 4096, 4096, 1, 16, 4),
     (40, 40, 8192, 1, 16, 16),

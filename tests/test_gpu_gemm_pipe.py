@@ -1,5 +1,5 @@
 """The pipelined GEMM tiles (1: 128x128, 9: 256x128, 16:
-64x64) against the
+64x64) and the 32x32 tile with K over the waves (17) against the
 oracle where they can go wrong: one K-step up to more than the ring holds,
 ragged M and N around a tile edge, M-tile counts that do not fill a group of
 four, split K, outputs the 16-byte stores do not fit, every epilogue, B as
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16])
+@pytest.mark.parametrize('tile', [1, 9, 16, 17])
 @pytest.mark.parametrize('kn', [False, True])
 @pytest.mark.parametrize('M,N,Kd,split', [
     (1, 8, 64, 1),            # one row, one 16-byte column chunk, one K-step
@@ -24,9 +24,12 @@ U = 2.0 ** -24
     (255, 120, 192, 1),       # one short of it
     (129, 136, 256, 1), (300, 520, 320, 1), (130, 128, 448, 1),   # around the 3- and 4-stage rings
     (1290, 392, 128, 1),      # 11 and 6 M-tiles: last group of four not full
+    (33, 40, 704, 1), (31, 24, 768, 1), (65, 72, 832, 1), (63, 56, 896, 1),   # 11 to 14 steps: each tail of the steps in fours
     (65, 72, 640, 1), (63, 56, 576, 1),   # around a 64 edge; 10 and 9 steps (odd and even tails of the step pairs)
     (300, 520, 1024, 4), (128, 256, 384, 3)])
 def test_pipe_tiles_tails(gpu, tile, kn, M, N, Kd, split):
+    if tile == 17 and (kn or split > 1):
+        pytest.skip('tile 17 takes B as [N][K] and no split')
     from chestnut import kernels as K
     print(f'[gemm] pipe tile {tile} kn={kn} {M}x{N}x{Kd} split {split}', flush=True)
     rng = np.random.default_rng(M + N + Kd + tile)
@@ -37,12 +40,14 @@ def test_pipe_tiles_tails(gpu, tile, kn, M, N, Kd, split):
     _gemm_check(C - b, A, B, transB=not kn, depth=Kd // 16 + 40)
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16])
+@pytest.mark.parametrize('tile', [1, 9, 16, 17])
 @pytest.mark.parametrize('kn,N,ldc', [(False, 201, 201), (False, 200, 203), (True, 200, 203)])
 @pytest.mark.parametrize('split', [1, 2])
 def test_pipe_tiles_without_16_byte_stores(gpu, tile, kn, N, ldc, split):
     """N odd, or a row pitch that is no multiple of 16 bytes: stored per
     element, and nothing outside [M][N] written."""
+    if tile == 17 and (kn or split > 1):
+        pytest.skip('tile 17 takes B as [N][K] and no split')
     from chestnut import _lib
     torch = gpu
     M, Kd = 150, 256
@@ -60,10 +65,12 @@ def test_pipe_tiles_without_16_byte_stores(gpu, tile, kn, N, ldc, split):
     assert (got[:, N:] == 7.0).all()
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16])
+@pytest.mark.parametrize('tile', [1, 9, 16, 17])
 @pytest.mark.parametrize('M,N,split', [(200, 264, 1), (200, 260, 1), (130, 264, 2)])
 @pytest.mark.parametrize('epi', [1, 2, 3, 4])
 def test_pipe_tiles_epilogues(gpu, tile, M, N, split, epi):
+    if tile == 17 and split > 1:
+        pytest.skip('tile 17 does not split K')
     from chestnut import kernels as K
     torch = gpu
     rng = np.random.default_rng(epi + N)
