@@ -47,6 +47,37 @@ __device__ __forceinline__ float xor_sum(float v) {
   return v + __shfl_xor(v, 32);
 }
 
+// Row-layout operands.  An MFMA fragment wants lane (g, r) to hold 16-byte chunk g
+// of row r.  A load in that order has neighbouring lanes on 16 different rows: 64
+// pieces of 16 bytes for the address unit, which bounds the kernel.  So rows are
+// loaded as they lie, RB bytes (128 or 64) of a row by RB / 16 neighbouring lanes,
+// and turned through LDS that the wave owns (no barrier): row-major there, chunk c
+// of a row at c ^ f(row), with f such that the 16 lanes served together hit 16
+// different 16-byte bank groups, in the writes and in the fragment reads alike.
+// Per launch against loads in fragment order (graph replays): 16 heads of 128 at
+// 512 tokens 11.6 -> 8.5 us, 32 of them 22.5 -> 16.6, 8 at 320 7.1 -> 5.4, 16 heads
+// of 64 at 512 7.0 -> 5.6, 8 at 256 4.2 -> 3.5, 4 at 64 2.6 either way.
+template <int N, int RB>
+__device__ __forceinline__ void rows_load(half8_t (&v)[N], const half_t* base, long stride, int lane) {
+  constexpr int CH = RB / 16;
+  const half_t* p = base + (lane / CH) * stride + (lane % CH) * 8;
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = *reinterpret_cast<const half8_t*>(p + (long)i * (64 / CH) * stride);
+}
+// byte of chunk c of a row; SWZ 0: fragments of 16 consecutive rows, 1: K's (rows 8q + 4p + i, q and i = 0..3)
+template <int RB, int SWZ>
+__device__ __forceinline__ int row_chunk(int row, int c) {
+  const int f = RB == 64 ? (row >> 2) & 3 : SWZ ? ((row >> 1) & 1) | ((row >> 2) & 6) : (row >> 1) & 7;
+  return row * RB + ((c ^ f) << 4);
+}
+template <int N, int RB, int SWZ>
+__device__ __forceinline__ void rows_to_lds(char* st, const half8_t (&v)[N], int lane) {
+  constexpr int CH = RB / 16;
+  const int r = lane / CH, c = lane % CH;
+#pragma unroll
+  for (int i = 0; i < N; ++i) *reinterpret_cast<half8_t*>(st + row_chunk<RB, SWZ>(i * (64 / CH) + r, c)) = v[i];
+}
+
 // Waves per workgroup for T = 64*NKT keys: every wave owns 32 or 64 keys.
 constexpr int att_waves(int nkt) { return nkt <= 4 ? 2 * nkt : nkt; }
 
@@ -55,13 +86,10 @@ constexpr int att_waves(int nkt) { return nkt <= 4 ? 2 * nkt : nkt; }
 // KB.  Otherwise the row layouts: qk [T][2d], vt [d][T].  There the two 16-key
 // tiles of a 32-key block take the keys 8q..8q+3 and 8q+4..8q+7 (q = 0..3) of
 // the block as their rows, so that the softmax leaves lane (g, r) the keys
-// 8g..8g+7: one 16-byte piece of a V^T row (in key order it is two 8-byte
-// pieces, twice the load instructions at half the bytes each; per launch, 16
-// heads of 128 at 512 tokens 16.1 -> 12.9 us, 12 at 384 12.7 -> 10.4, 8 heads of
-// 64 at 512 9.1 -> 7.4, at 256 5.7 -> 4.8).  Loading whole 128-byte lines and
-// exchanging halves between lanes, or spreading a head over the XCDs, measured
-// no faster (12.8 and 13.6 us).  All of a wave's loads (Q, its K, its V) are
-// issued at entry, before any MFMA.
+// 8g..8g+7: one 16-byte chunk of a V^T row.  The rows reach the fragments
+// through LDS (rows_load).  Spreading a head over the XCDs measured slower
+// (13.6 us against 12.9 with loads in fragment order).  All of a wave's loads
+// (Q, its K, its V) are issued at entry, before any MFMA.
 // QT: 16-query tiles per workgroup (2: 32 queries; 1: 16, twice the
 // workgroups for short sequences that would leave most CUs idle).
 // OTW > 0: the output projection rides along.  The workgroup's normalised
@@ -98,7 +126,13 @@ __global__ __launch_bounds__(64 * att_waves(NKT)) void attention_kernel(const ha
   constexpr bool P16 = OTW > 0;
   typedef std::conditional_t<P16, half_t, float> part_t;
   constexpr int OP = P16 ? HD + 8 : HD + 4;
-  __shared__ __attribute__((aligned(16))) part_t part[WAVES][QB][OP];
+  // row layout: each wave's area for turning K, Q and V^T into fragments, in the
+  // same memory (the partial outputs come after the last fragment read)
+  constexpr int TURN = FRAG ? 0 : (KPW > QB ? KPW : QB) * HD * 2;
+  constexpr int SMEM = WAVES * QB * OP * (int)sizeof(part_t) > WAVES * TURN ? WAVES * QB * OP * (int)sizeof(part_t)
+                                                                            : WAVES * TURN;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
+  part_t (*const part)[QB][OP] = reinterpret_cast<part_t (*)[QB][OP]>(smem);
   __shared__ float mrow[WAVES][QB], lrow[WAVES][QB];
   constexpr int KSO = HD / 32;       // k-steps of the O-projection
   constexpr int OBP = HD + 8;        // f16 output row pitch in LDS (16-byte rows)
@@ -117,6 +151,9 @@ __global__ __launch_bounds__(64 * att_waves(NKT)) void attention_kernel(const ha
 
   // ---- all loads up front ----
   half8_t qf[QT][KS], kf[KT][KS], vb[KB][CT];
+  constexpr int VRB = KPW * 2, NVL = HD * VRB / 1024;   // row layout: V^T rows of KPW keys, their loads
+  half8_t vl[FRAG ? 1 : NVL];
+  char* const turn = reinterpret_cast<char*>(smem) + wave * TURN;
   if constexpr (FRAG) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
@@ -137,24 +174,37 @@ __global__ __launch_bounds__(64 * att_waves(NKT)) void attention_kernel(const ha
         vb[kb][ct] = *reinterpret_cast<const half8_t*>(
             vt + ((((long)h * (HD / 16) + ct) * (T / 32) + kw0 / 32 + kb) * 64 + lane) * 8);
   } else {
+    // halves of 64 head dims: 8 rows of 128 bytes per load
+    constexpr int HH = HD / 64, NK = KPW / 8, NQ = QB / 8;
+    half8_t kl[HH][NK], ql[HH][NQ];
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      // tile row r is key (r / 4) * 8 + (kt % 2) * 4 + r % 4 of its 32-key block
-      const int key = kw0 + (kt >> 1) * 32 + (r16 >> 2) * 8 + (kt & 1) * 4 + (r16 & 3);
-      const half_t* kr = qk + (long)key * ldq + d + h * HD + g * 8;
+    for (int f = 0; f < HH; ++f) rows_load<NK, 128>(kl[f], qk + (long)kw0 * ldq + d + h * HD + f * 64, ldq, lane);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kf[kt][ks] = *reinterpret_cast<const half8_t*>(kr + ks * 32);
-    }
+    for (int f = 0; f < HH; ++f) rows_load<NQ, 128>(ql[f], qk + (long)q0 * ldq + h * HD + f * 64, ldq, lane);
+    rows_load<NVL, VRB>(vl, vt + (long)h * HD * T + kw0, T, lane);
+#pragma unroll
+    for (int f = 0; f < HH; ++f) rows_to_lds<NK, 128, 1>(turn + f * KPW * 128, kl[f], lane);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)   // tile row r is key (r / 4) * 8 + (kt % 2) * 4 + r % 4 of its 32-key block
+        kf[kt][ks] = *reinterpret_cast<const half8_t*>(
+            turn + (ks >> 1) * KPW * 128 +
+            row_chunk<128, 1>((kt >> 1) * 32 + (r16 >> 2) * 8 + (kt & 1) * 4 + (r16 & 3), (ks & 1) * 4 + g));
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int f = 0; f < HH; ++f) rows_to_lds<NQ, 128, 0>(turn + f * QB * 128, ql[f], lane);
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
-        qf[qt][ks] = *reinterpret_cast<const half8_t*>(qk + (long)(q0 + qt * 16 + r16) * ldq + h * HD + ks * 32 + g * 8);
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-        vb[kb][ct] = *reinterpret_cast<const half8_t*>(vt + (long)(h * HD + ct * 16 + r16) * T + kw0 + kb * 32 + 8 * g);
+        qf[qt][ks] = *reinterpret_cast<const half8_t*>(turn + (ks >> 1) * QB * 128 +
+                                                       row_chunk<128, 0>(qt * 16 + r16, (ks & 1) * 4 + g));
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
   }
   // W_o fragments (MFMA A operand: row n = output feature, 8 k of head h's columns)
   half8_t wf[OTW > 0 ? OTW : 1][KSO];
@@ -207,6 +257,18 @@ __global__ __launch_bounds__(64 * att_waves(NKT)) void attention_kernel(const ha
     }
   }
 
+  if constexpr (!FRAG) {
+    rows_to_lds<NVL, VRB, 0>(turn, vl, lane);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        vb[kb][ct] = *reinterpret_cast<const half8_t*>(turn + row_chunk<VRB, 0>(ct * 16 + r16, kb * 4 + g));
+    // part overlaps the turning areas: every wave is past its V reads
+    wait_vm_lgkm0<0>();
+    lds_barrier();
+  }
   // ---- 3. O_w = e V over this wave's keys ----
   if constexpr (P16) {
     // O_w^T = V^T e^T (operands swapped: lane (g, r16) ends with head dims
