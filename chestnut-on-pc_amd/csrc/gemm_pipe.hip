@@ -1,6 +1,7 @@
 // f16-input / f32-accumulate GEMM for products large enough to keep the matrix
-// cores busy: 128x128 and 256x128 tiles, B as [N][K] or [K][N], one
-// workgroup per CU, the K loop software-pipelined across its barrier.
+// cores busy: 128x128 and 256x128 tiles with one workgroup per CU, and 64x64
+// tiles for products with few of those; B as [N][K] or [K][N]; the K loop
+// software-pipelined across its barrier.
 //
 // What bounds it.  A wave issues in order and an MFMA occupies the matrix core
 // for 32 cycles, so every instruction that makes a wave wait between two MFMAs
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 && S <= 4 ? 2 : 1) void ge
 
   // NCH accumulators per product, each taking every NCH-th k-slice: a chain of
   // roundings is that much shorter (relative error at K = 4096: one chain 4.1e-7,
-  // two 2.9e-7, eight 1.6e-7).  The 64x64 tile, whose products leave room for
+  // two 2.9e-7).  The 64x64 tile, whose products leave room for
   // eight, then needs no split of K to be as exact as a split one was.
   constexpr int NCH = NM == 1 ? 8 : 2;
   float16_t acc[NCH][FM][1][FN];
