@@ -24,7 +24,7 @@
 // LDS-DMA load in flight has landed (vmcnt(0)), which serialises the ring; the
 // reads of a slice are therefore one asm block that ends with their own wait.
 //
-// Measured on one box, us per call (TFLOP/s), before = the 128x128 tile of
+// Measured on one card, us per call (TFLOP/s), before = the 128x128 tile of
 // gemm.hip with two K-groups:
 //   4096x4096x4096, B [N][K]: 245 (560) -> 126 (1090) on 256x128 (128x128 here 150)
 //   4096x4096x4096, B [K][N]: 245 (560) -> 133 (1030) on 256x128 (128x128 158)
