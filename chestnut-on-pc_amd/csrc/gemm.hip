@@ -1374,8 +1374,14 @@ size_t gemm_plan(GemmDesc& d) {
     const long t = (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch;
     if (t < 64) bm = bn = 64;
     d.tile = bm == 128 ? (bn == 128 ? 1 : 2) : (bn == 128 ? 3 : 4);
-    if (d.tile == 1 && d.split <= 1) d.tile = tile_of_many(d);
-    if (!d.b_kn && d.tile >= 2 && d.tile <= 4 && d.split <= 1) {
+    // the tiles chosen from here on (9, 16, 17) serve the row-major f32, f16 and
+    // residual outputs; the frame plan's other epilogues and the implicit
+    // convolution stay on 1-4
+    const bool rows = d.conv_c == 0 && !d.c_nm &&
+                      (d.epi == EPI_F32 || d.epi == EPI_F16_BIAS || d.epi == EPI_F16_BIAS_RELU ||
+                       d.epi == EPI_F16_BIAS_GELU || d.epi == EPI_F32_RESID);
+    if (rows && d.tile == 1 && d.split <= 1) d.tile = tile_of_many(d);
+    if (rows && !d.b_kn && d.tile >= 2 && d.tile <= 4 && d.split <= 1) {
       // one 64-wide dimension and a K too short to split: 64x64 keeps twice the
       // CUs busy (128x8192x512 on 64x128 7.6, on 64x64 5.5 us)
       if (d.K / BK < 16) d.tile = 4;

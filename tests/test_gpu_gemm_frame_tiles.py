@@ -1,0 +1,39 @@
+"""Frame plans with their GEMMs on tiles other than the plan's own, through the
+spec's gemm_config, against the oracle within the plan tolerance."""
+import numpy as np
+import pytest
+
+from chestnut import Engine
+from chestnut import spec as S
+from chestnut import tune as TU
+from oracle import model as OM
+from test_gpu_engine import REL, frame_inputs, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def frames_match(sp, cfg):
+    """Two recurrent frames of the spec under a gemm_config, against the oracle."""
+    w = S.make_weights(sp)
+    orc = OM.OracleModel(sp, w, acc=np.float64)
+    rng = np.random.default_rng(7)
+    print(f'[frame] {sp["name"]} {cfg}', flush=True)
+    with Engine(dict(sp, gemm_config=cfg), weights=w) as eng:
+        hs = None
+        for f, (warped, packed) in enumerate(frame_inputs(rng, sp['name'], 2)):
+            if hs is not None:
+                packed[12:] = hs
+            out = eng.run_frame(warped, packed)
+            ref = orc.run_frame(warped, packed)
+            for name, sl in eng.out_slices.items():
+                e = rel_err(out[sl], ref[sl])
+                assert e <= REL, (f, name, e)
+            hs = out[eng.out_slices['hidden_state']]
+
+
+@pytest.mark.parametrize('spec', ['tiny', 'driving_39m'])
+def test_every_gemm_at_tile_code_0(gpu, spec):
+    """The automatic tile and split of every GEMM of the plan, the
+    O-projection on a launch of its own among them."""
+    sp = dict(S.get_spec(spec), n_layers=2, fuse_oproj=0)
+    frames_match(sp, TU.config_for(sp, {fam: (0, 0) for fam in TU.shapes(sp)}))
