@@ -7,7 +7,8 @@
 // The kernels here and in gemm_pipe.hip work tile by tile instead:
 //   * gemm_pipe_kernel (gemm_pipe.hip; tile codes 1, 9 and 16): the K loop
 //     software-pipelined across its barrier, B as [N][K] or [K][N];
-//   * gemm_dma_kernel (tile codes 2-8, 10, 15; 1 for an implicit convolution):
+//   * gemm_dma_kernel (tile codes 2-8, 10, 15; 1 for an implicit convolution, 1
+//     and 9 for the QKV epilogues):
 //     A and B tiles go straight from global memory into an S-stage LDS ring with
 //     global_load_lds_dwordx4, XOR-swizzled for conflict-free MFMA operand
 //     reads; v_mfma_f32_32x32x16_f16 on a grid of 64x64 wave tiles (32x96 on
@@ -1111,7 +1112,8 @@ void launch_tile(const GemmParams& p, hipStream_t s) {
 
 // tile codes (BM x BN): 1 128x128, 2 128x64, 3 64x128, 4 64x64.
 //   1, 9 (256x128), 16 (64x64): the pipelined kernel (gemm_pipe.hip), [N][K] or
-//        [K][N] B (implicit conv with tile 1: the LDS-DMA kernel);
+//        [K][N] B (implicit conv with tile 1, the QKV epilogues with 1 and 9:
+//        the LDS-DMA kernel, as 2-4 and with 8 waves in one K-group);
 //   2-4: LDS-DMA kernel with two K-groups (8 waves) when K per split is a
 //        multiple of 128, else one group;  5-8: LDS-DMA, one group, 5 128x128
 //        (a [K][N] B is first transposed into the workspace);
@@ -1138,12 +1140,24 @@ void launch_epi(int tile, const GemmParams& p, hipStream_t s) {
     }
     throw Error("gemm: tile 15 (32x64) takes B as [N][K] only");
   }
+  if (tile == 9) {   // 256x128, 8 waves of 64x64, one K-group, 3-stage ring (3 x 48 KB): the QKV epilogues
+    if constexpr (!BKN && (EPI == EPI_QKV || EPI == EPI_QKV_FRAG)) {
+      CK_LAUNCH((gemm_dma_kernel<256, 128, 3, 1, EPI, 8>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(512), 0, s, p);
+      CK_LAUNCHED("gemm_dma");
+      return;
+    }
+    throw Error("gemm: tile 9 (256x128) on the LDS-DMA kernel serves the QKV epilogues only");
+  }
   if (!BKN && tile < 10) {
     const bool kg2 = c <= 4 && p.kps % (2 * BK) == 0;
     switch (c > 4 ? c - 4 : c) {
-      case 1:
-        CK_LAUNCH((gemm_dma_kernel<128, 128, 5, 1, EPI>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(256), 0, s, p);
-        CK_LAUNCHED("gemm_dma");
+      case 1:   // two K-groups (tile 1) for the QKV epilogues only: gemm_pipe_kernel has the others' tile 1
+        if constexpr (EPI == EPI_QKV || EPI == EPI_QKV_FRAG) {
+          launch_dma_tile<128, 128, EPI>(p, kg2, s);
+        } else {
+          CK_LAUNCH((gemm_dma_kernel<128, 128, 5, 1, EPI>), dim3(p.Mt * p.Nt * p.split * p.batch), dim3(256), 0, s, p);
+          CK_LAUNCHED("gemm_dma");
+        }
         break;
       case 2: launch_dma_tile<128, 64, EPI>(p, kg2, s); break;
       case 3: launch_dma_tile<64, 128, EPI>(p, kg2, s); break;
@@ -1215,8 +1229,11 @@ void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s) {
 }
 
 // The tiles of the pipelined kernel (gemm_pipe.hip): 1 (128x128), 9 (256x128)
-// and 16 (64x64), for everything but the implicit convolution.
-bool tile_pipe(const GemmDesc& d) { return (d.tile == 1 || d.tile == 9 || d.tile == 16) && d.conv_c == 0; }
+// and 16 (64x64), for everything but the implicit convolution and the QKV
+// epilogues, whose tiles 1 and 9 stay on the LDS-DMA kernel.
+bool tile_pipe(const GemmDesc& d) {
+  return (d.tile == 1 || d.tile == 9 || d.tile == 16) && d.conv_c == 0 && d.epi != EPI_QKV && d.epi != EPI_QKV_FRAG;
+}
 
 // Tiles that take a [K][N] B as it lies (no transpose pass, no workspace for
 // it): the pipelined ones read it transposed out of LDS, tile 2 brings it in
@@ -1398,8 +1415,6 @@ size_t gemm_plan(GemmDesc& d) {
                               (d.epi == EPI_F32 || d.epi == EPI_F16_BIAS || d.epi == EPI_F16_BIAS_RELU ||
                                d.epi == EPI_F16_BIAS_GELU || d.epi == EPI_F32_RESID)),
              "gemm: tile 17 (32x32, K over the waves) takes B as [N][K], split 1 and the f32, f16 and residual epilogues");
-  // the QKV epilogues run on the LDS-DMA kernel's 128x128 tile
-  if ((d.epi == EPI_QKV || d.epi == EPI_QKV_FRAG) && (d.tile == 1 || d.tile == 9)) d.tile = 5;
   CK_REQUIRE(d.tile != 15 || !d.b_kn, "gemm: tile 15 (32x64) takes B as [N][K]");
   CK_REQUIRE(d.tile != 10 || (d.epi == EPI_QKV_FRAG && !d.b_kn && d.conv_c == 0),
              "gemm: tile 10 (128x96) serves the QKV fragment epilogue only");

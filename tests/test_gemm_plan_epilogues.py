@@ -100,3 +100,12 @@ def test_tile_code_0_of_the_39m_entries(planner):
 def test_row_major_outputs_keep_the_small_and_large_tiles(planner, epi):
     got = planner([row(200, 520, 2048, epi), row(4096, 4096, 4096, epi), row(1000, 1000, 1024, epi)])
     assert [g[:2] for g in got] == [(17, 1), (9, 1), (16, 1)]
+
+
+@pytest.mark.parametrize('epi', ['qkv', 'qkv_frag'])
+def test_an_asked_qkv_tile_stays(planner, epi):
+    """Tile 1 (two K-groups) and tile 9 (256x128) are kernels of their own for
+    the QKV epilogues, not other names of tile 5."""
+    tiles = [1, 2, 3, 4, 5, 8, 9, 15] + ([10] if epi == 'qkv_frag' else [])
+    got = planner([row(512, 6144, 2048, epi, head_dim=128, tile=t, split=1) for t in tiles])
+    assert [g[:2] for g in got] == [(t, 1) for t in tiles]

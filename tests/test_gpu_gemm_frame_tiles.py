@@ -37,3 +37,12 @@ def test_every_gemm_at_tile_code_0(gpu, spec):
     O-projection on a launch of its own among them."""
     sp = dict(S.get_spec(spec), n_layers=2, fuse_oproj=0)
     frames_match(sp, TU.config_for(sp, {fam: (0, 0) for fam in TU.shapes(sp)}))
+
+
+@pytest.mark.parametrize('spec', ['tiny', 'driving_39m'])
+@pytest.mark.parametrize('tile', [1, 9])
+def test_qkv_on_128_and_256_row_tiles(gpu, spec, tile):
+    """Two K-groups of 128x128 (tile 1) and 256x128 (tile 9), M below and at
+    their rows."""
+    sp = dict(S.get_spec(spec), n_layers=2)
+    frames_match(sp, TU.config_for(sp, {'qkv': (tile, 1)}))
