@@ -1213,21 +1213,6 @@ void launch_reduce(const GemmParams& p, hipStream_t s, const GemvRider* rider = 
   CK_LAUNCHED("splitk_reduce_gemv");
 }
 
-// The split-K reduce of an epilogue (EPI_PARTIALS leaves its partials to the
-// LayerNorm that consumes them).
-void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s) {
-  switch (epi) {
-    case EPI_F32: launch_reduce<EPI_F32>(p, s); break;
-    case EPI_F16_BIAS: launch_reduce<EPI_F16_BIAS>(p, s); break;
-    case EPI_F16_BIAS_RELU: launch_reduce<EPI_F16_BIAS_RELU>(p, s); break;
-    case EPI_F16_BIAS_GELU: launch_reduce<EPI_F16_BIAS_GELU>(p, s); break;
-    case EPI_F32_RESID: launch_reduce<EPI_F32_RESID>(p, s); break;
-    case EPI_EMBED: launch_reduce<EPI_EMBED>(p, s); break;
-    case EPI_QKV: launch_reduce<EPI_QKV>(p, s); break;
-    default: break;
-  }
-}
-
 // The tiles of the pipelined kernel (gemm_pipe.hip): 1 (128x128), 9 (256x128)
 // and 16 (64x64), for everything but the implicit convolution and the QKV
 // epilogues, whose tiles 1 and 9 stay on the LDS-DMA kernel.
@@ -1364,6 +1349,13 @@ bool small_tiles_win(const GemmDesc& d) {
   const float other = 3.f + 0.3f * (float)(ks / s) + (s > 1 ? 3.5f + 0.1f * (float)s : 0.f);
   return t17 < other;
 }
+
+// Defined behind launch_gemm: the compiler lays kernels out in the order of their
+// first use, and launch_gemm uses the implicit-conv kernels and the reduces of
+// their epilogue side by side, as the frame's conv stem runs them.  With the
+// reduces of every epilogue first, 39M plan replays took 182.4 us instead of
+// 181.4 (medians of six processes each, in turn); the instructions are the same.
+void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s);
 
 }  // namespace
 
@@ -1587,5 +1579,24 @@ void launch_gemm(GemmDesc d, hipStream_t s) {
   }
   if (d.split > 1 && !p.pair) launch_reduce_epi(d.epi, p, s);
 }
+
+namespace {
+
+// The split-K reduce of an epilogue (EPI_PARTIALS leaves its partials to the
+// LayerNorm that consumes them).
+void launch_reduce_epi(int epi, const GemmParams& p, hipStream_t s) {
+  switch (epi) {
+    case EPI_F32: launch_reduce<EPI_F32>(p, s); break;
+    case EPI_F16_BIAS: launch_reduce<EPI_F16_BIAS>(p, s); break;
+    case EPI_F16_BIAS_RELU: launch_reduce<EPI_F16_BIAS_RELU>(p, s); break;
+    case EPI_F16_BIAS_GELU: launch_reduce<EPI_F16_BIAS_GELU>(p, s); break;
+    case EPI_F32_RESID: launch_reduce<EPI_F32_RESID>(p, s); break;
+    case EPI_EMBED: launch_reduce<EPI_EMBED>(p, s); break;
+    case EPI_QKV: launch_reduce<EPI_QKV>(p, s); break;
+    default: break;
+  }
+}
+
+}  // namespace
 
 }  // namespace ck
