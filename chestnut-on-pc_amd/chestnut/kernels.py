@@ -21,7 +21,16 @@ from ._lib import check, lib
 # device queries torch itself uses, plain integers for pointers, and the GEMM
 # planner's answer remembered by sizes (LayerNorm of 64 x 128: 10.8 -> 6.7 us per
 # call, of which the raw C call is 4.0 and the output's allocation 1.1).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+try:
+    from torch._C import _cuda_getCurrentRawStream as _raw_stream
+    from torch._C import _cuda_getDevice as _device
+except ImportError:   # a torch without GPU support: the argument checks still run
+
+    def _raw_stream(dev):
+        return torch.cuda.current_stream(dev).cuda_stream
+
+    def _device():
+        return torch.cuda.current_device()
 
 
 def _ptr(t):
@@ -63,7 +72,7 @@ def _validate(*args):
     for placement on the current CUDA device, whose index is returned."""
     first = args[0][0]
     dev = first.get_device() if type(first) is torch.Tensor else -1
-    if dev < 0 or dev != torch._C._cuda_getDevice():
+    if dev < 0 or dev != _device():
         return _validate_each(args)
     for a in args:
         t = a[0]

@@ -4,6 +4,10 @@ that disagrees with the sizes derived from the other operands, a
 non-contiguous view, a tensor that is not on the current CUDA device.
 Shape checks run before the device check, so on the CPU every argument's
 check is reachable with CPU tensors."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -81,3 +85,19 @@ def test_well_formed_cpu_tensors_stop_at_the_device_check():
         K.gemv(z(8, 64, dtype=f16), z(64), bias=z(8), out=z(8))
     with pytest.raises(ValueError, match='must be a CUDA tensor'):
         K.gemm_epi(z(16, 64, dtype=f16), z(32, 64, dtype=f16), z(32), 3, z(16, 32, dtype=f16))
+
+
+def test_checks_run_on_a_torch_without_gpu_support():
+    """Such a torch has no stream or device query: the module imports and its
+    checks answer as ever."""
+    prog = (f'import sys; sys.path.insert(0, {os.path.dirname(os.path.dirname(K.__file__))!r})\n'
+            'import torch\n'
+            'del torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice\n'
+            'from chestnut import kernels as K\n'
+            'try:\n'
+            '    K.layernorm(torch.zeros(4, 128), torch.zeros(128), torch.zeros(128))\n'
+            'except ValueError as e:\n'
+            '    print(e)\n')
+    r = subprocess.run([sys.executable, '-c', prog], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    assert 'x must be a CUDA tensor' in r.stdout
