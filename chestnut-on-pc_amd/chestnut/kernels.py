@@ -99,11 +99,21 @@ def gemv(W, x, bias=None, act=0, rows_per_wg=0, out=None):
     return y
 
 
-@functools.lru_cache(maxsize=256)
-def gemm_workspace(M, N, K, b_kn, tile=0, split_k=0):
+def _plan(M, N, K, b_kn, tile, split_k):
     t, s, nb = ctypes.c_int(tile), ctypes.c_int(split_k), ctypes.c_size_t()
-    check(lib().ck_gemm_workspace(M, N, K, 1 if b_kn else 0, ctypes.byref(t), ctypes.byref(s), ctypes.byref(nb)))
+    check(lib().ck_gemm_workspace(M, N, K, b_kn, ctypes.byref(t), ctypes.byref(s), ctypes.byref(nb)))
     return t.value, s.value, nb.value
+
+
+_cached_plan = functools.lru_cache(maxsize=256)(_plan)
+
+
+def gemm_workspace(M, N, K, b_kn, tile=0, split_k=0):
+    """(tile, split, workspace bytes) of the planner.  Remembered for plain
+    integers only: a float equal to one is refused here as by the library, and
+    an object that can change (a 0-d tensor) is asked for its value each time."""
+    plan = _cached_plan if type(M) is type(N) is type(K) is type(tile) is type(split_k) is int else _plan
+    return plan(M, N, K, 1 if b_kn else 0, tile, split_k)
 
 
 def _workspace(ws, nb, device):
@@ -125,7 +135,8 @@ def gemm(A, B, b_kn=True, bias=None, tile=0, split_k=0, out=None, workspace=None
     N = B.shape[1] if b_kn else B.shape[0]
     dev = _validate((A, torch.float16, 'A'), (B, torch.float16, 'B', (K, N) if b_kn else (N, K)),
                     (bias, torch.float32, 'bias', (N,)), (out, torch.float32, 'out', (M, N)))
-    tile, split_k, nb = gemm_workspace(M, N, K, b_kn, tile, split_k)
+    plan = _cached_plan if type(tile) is type(split_k) is int else _plan   # as gemm_workspace
+    tile, split_k, nb = plan(M, N, K, 1 if b_kn else 0, tile, split_k)
     C = out if out is not None else torch.empty(M, N, dtype=torch.float32, device=A.device)
     ws = _workspace(workspace, nb, A.device)
     check(lib().ck_gemm(A.data_ptr(), B.data_ptr(), C.data_ptr(), _ptr(bias), M, N, K, K, N if b_kn else K, N,
@@ -150,7 +161,8 @@ def gemm_epi(A, W, bias, epi, out, tile=0, split_k=0):
         raise ValueError('out is required')
     dev = _validate((A, torch.float16, 'A'), (W, torch.float16, 'W', (N, K)), (bias, torch.float32, 'bias', (N,)),
                     (out, _EPI_OUT[epi], 'out', (M, N)))
-    tile, split_k, nb = gemm_workspace(M, N, K, False, tile, split_k)
+    plan = _cached_plan if type(tile) is type(split_k) is int else _plan   # as gemm_workspace
+    tile, split_k, nb = plan(M, N, K, 0, tile, split_k)
     ws = _workspace(None, nb, A.device)
     check(lib().ck_gemm_epi(A.data_ptr(), W.data_ptr(), out.data_ptr(), _ptr(bias), M, N, K, K, K, N, epi, tile,
                             split_k, _ptr(ws), nb, _raw_stream(dev)))

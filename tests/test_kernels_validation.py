@@ -101,3 +101,17 @@ def test_checks_run_on_a_torch_without_gpu_support():
     r = subprocess.run([sys.executable, '-c', prog], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
     assert 'x must be a CUDA tensor' in r.stdout
+
+
+def test_gemm_workspace_remembers_plain_integers_only():
+    want = K.gemm_workspace(256, 256, 256, False, 4, 2)
+    assert want == (4, 2, 4 * 2 * 256 * 256)
+    assert K.gemm_workspace(256, 256, 256, [], 4, 2) == want and K.gemm_workspace(256, 256, 256, False, 4, 2) == want
+    with pytest.raises(TypeError):
+        K.gemm_workspace(256, 256, 256, False, 4.0, 2)
+    with pytest.raises(TypeError):
+        K.gemm_workspace(256, 256, 256, False, 4, 2.0)
+    split = torch.tensor(2)
+    assert K.gemm_workspace(256, 256, 256, False, 4, split) == want
+    split.fill_(4)
+    assert K.gemm_workspace(256, 256, 256, False, 4, split) == (4, 4, 4 * 4 * 256 * 256)
