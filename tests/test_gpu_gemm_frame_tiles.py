@@ -46,3 +46,23 @@ def test_qkv_on_128_and_256_row_tiles(gpu, spec, tile):
     their rows."""
     sp = dict(S.get_spec(spec), n_layers=2)
     frames_match(sp, TU.config_for(sp, {'qkv': (tile, 1)}))
+
+
+@pytest.mark.parametrize('spec,split', [('tiny', 1), ('tiny', 2), ('driving_39m', 4)])
+@pytest.mark.parametrize('tile', [1, 9, 16])
+def test_partials_and_embedding_on_the_pipelined_tiles(gpu, spec, split, tile):
+    """The split-K partials that the next LayerNorm adds (O-projection, MLP
+    down) and the embedding's epilogue on gemm_pipe_kernel."""
+    sp = dict(S.get_spec(spec), n_layers=2, fuse_oproj=0)
+    frames_match(sp, TU.config_for(sp, {'o': (tile, split), 'down': (tile, split), 'embed': (tile, 1)}))
+
+
+@pytest.mark.parametrize('tile,split', [(1, 1), (9, 1), (16, 1), (17, 1), (9, 3), (16, 3)])
+def test_batched_stem_on_the_pipelined_and_small_tiles(gpu, tile, split):
+    """Two images per launch: stem layer 0, and the last layer, which the tiles
+    without an implicit-conv A take through its patch matrix (K = 576)."""
+    sp = dict(S.get_spec('tiny'), n_layers=2)
+    cfg = {'stem0.conv': [tile, 1]}
+    if tile != 1:
+        cfg['stem4.conv'] = [tile, split]
+    frames_match(sp, cfg)

@@ -93,3 +93,34 @@ def test_pipe_tiles_epilogues(gpu, tile, M, N, split, epi):
     # one f16 rounding of an f32 value within reassociation noise: at most one ulp apart
     ulp = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
     assert np.all(np.abs(host(out).astype(np.float64) - ref) <= ulp + 1e-7)
+
+
+@pytest.mark.parametrize('tile', [1, 9, 16])
+@pytest.mark.parametrize('epi,M,N', [(4, 16400, 32776), (1, 32792, 32776)])
+def test_pipe_tiles_output_of_2_gib(gpu, tile, epi, M, N):
+    """Outputs whose offsets do not fit the 32-bit buffer stores leave by
+    non-temporal ones: the first and last rows, the rows around 2 GiB and some
+    between, against 64-bit sums."""
+    from chestnut import kernels as K
+    torch = gpu
+    Kd, el = 64, 4 if epi == 4 else 2
+    assert el * M * N > 1 << 31
+    g = torch.Generator(device='cuda')
+    g.manual_seed(M + tile)
+    A = (torch.randn(M, Kd, generator=g, device='cuda') / 8).half()
+    W = (torch.randn(N, Kd, generator=g, device='cuda') / 8).half()
+    b = torch.randn(N, generator=g, device='cuda')
+    at = (1 << 31) // (el * N)
+    rows = torch.tensor(sorted({0, 1, 255, 256, M // 3, at - 1, at, at + 1, M - 2, M - 1}), device='cuda')
+    print(f'[gemm] 2 GiB output, tile {tile} epi {epi} {M}x{N}', flush=True)
+    out = torch.zeros(M, N, dtype=torch.float32 if epi == 4 else torch.float16, device='cuda')
+    if epi == 4:
+        out[rows] = 3.0
+    K.gemm_epi(A, W, b, epi, out, tile=tile, split_k=1)
+    Wt = W.double().t().contiguous()
+    ref = A[rows].double() @ Wt + b.double() + (3.0 if epi == 4 else 0.0)
+    scale = A[rows].double().abs() @ Wt.abs() + b.double().abs() + 3.0
+    err = (Kd // 16 + 40) * U * scale + (0 if epi == 4 else 2.0 ** -11 * ref.abs() + 2.0 ** -25)
+    assert bool(((out[rows].double() - ref).abs() <= err).all())
+    # and every other row was written: none is left as it was
+    assert bool((out.count_nonzero(dim=1) > N // 2).all())

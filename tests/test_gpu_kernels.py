@@ -246,13 +246,12 @@ def test_gemm_split2_on_concurrent_streams(gpu):
                                           (300, 384, 1024, 4), (64, 128, 256, 2), (300, 192, 768, 1),
                                           (64, 128, 1536, 2)])
 def test_gemm_kn_paths(gpu, tile, M, N, Kd, split):
-    """[K][N] B: with N a multiple of 128 the two-K-group 128x128 LDS-DMA
-    tile (1, and 0 when it picks it) and the 8-wave 256x128 tile (9) stream
-    it into LDS as it is and read their MFMA fragments transposed; the
-    128x64 tile (2) with N a multiple of 64 and K per split a multiple of 384
-    loads it through registers and writes it to LDS in the [N][K] layout;
-    otherwise the LDS-DMA tiles (2, 4, 5, 9, ...) transpose it into the
-    workspace first, and the register-staged tiles (11, 13) transpose it in
+    """[K][N] B: tiles 1 (128x128), 9 (256x128) and what tile 0 resolves to here
+    (16, 64x64) stream it into LDS as it is and read their MFMA fragments
+    transposed (gemm_pipe.hip); the 128x64 tile (2) with N a multiple of 64 and
+    K per split a multiple of 384 loads it through registers and writes it to
+    LDS in the [N][K] layout; otherwise the LDS-DMA tiles (2, 4, 5) transpose it
+    into the workspace first, and the register-staged tiles (11, 13) transpose it in
     registers; ragged M and N."""
     from chestnut import kernels as K
     rng = np.random.default_rng(M + N + tile)
@@ -320,6 +319,38 @@ def test_gemm_epilogues(gpu, epi, N, tile):
     # f16 rounding of an f32 value within reassociation noise: at most one f16 ulp apart
     ulp = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
     assert np.all(np.abs(got - ref) <= ulp + 1e-7)
+
+
+@pytest.mark.parametrize('tile', [2, 3, 4, 8])
+# K per split of whole pairs of K-steps (two K-groups on tiles 2-4) and not, with
+# and without a split; N = 196 takes the per-element epilogue
+@pytest.mark.parametrize('N,Kd,split', [(200, 256, 1), (196, 256, 1), (200, 192, 1), (200, 512, 2), (196, 384, 2)])
+@pytest.mark.parametrize('epi', [1, 2, 3, 4])
+def test_gemm_epilogues_lds_dma_tiles(gpu, epi, N, Kd, split, tile):
+    from chestnut import kernels as K
+    torch = gpu
+    rng = np.random.default_rng(10 * epi + tile)
+    M = 96
+    A = (rng.standard_normal((M, Kd)) / 8).astype(np.float16)
+    W = (rng.standard_normal((N, Kd)) / 8).astype(np.float16)
+    b = rng.standard_normal(N).astype(np.float32)
+    acc = OK.gemm(A, W, transB=True) + b
+    scale = np.abs(A.astype(np.float64)) @ np.abs(W.astype(np.float64)).T + np.abs(b)
+    if epi == 4:
+        C0 = rng.standard_normal((M, N)).astype(np.float32)
+        out = dev(torch, C0.copy())
+        K.gemm_epi(dev(torch, A), dev(torch, W), dev(torch, b), 4, out, tile=tile, split_k=split)
+        assert np.all(np.abs(host(out) - (C0 + acc)) <= (Kd // 16 + 40) * U * (scale + np.abs(C0)))
+        return
+    out = torch.empty(M, N, dtype=torch.float16, device='cuda')
+    K.gemm_epi(dev(torch, A), dev(torch, W), dev(torch, b), epi, out, tile=tile, split_k=split)
+    ref = {1: lambda v: v, 2: lambda v: np.maximum(v, 0), 3: OK.gelu}[epi](acc)
+    # one f16 rounding (half an ulp) of an f32 value within its summation error; the
+    # GELU's derivative is at most 1.13, and its exponential (an exponent below 40 in
+    # f32, an error of 3 roundings) and reciprocal add less than 1e-5 of the value
+    ulp = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
+    err = 1.2 * (Kd // 16 + 40) * U * scale + 1e-5 * np.abs(ref)
+    assert np.all(np.abs(host(out).astype(np.float64) - ref) <= 0.5 * ulp + err)
 
 
 # ------------------------------------------------------- packing / image ----
