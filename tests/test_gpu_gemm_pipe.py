@@ -16,9 +16,13 @@ pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16, 17])
-@pytest.mark.parametrize('kn', [False, True])
-@pytest.mark.parametrize('M,N,Kd,split', [
+def tiles_for(shapes, kn_of, split_of):
+    """(tile, *shape) of every tile and shape that go together: tile 17 takes B as
+    [N][K] and no split."""
+    return [(t, *s) for s in shapes for t in (1, 9, 16, 17) if t != 17 or not kn_of(s) and split_of(s) == 1]
+
+
+TAILS = [
     (1, 8, 64, 1),            # one row, one 16-byte column chunk, one K-step
     (257, 264, 128, 1),       # one past the 256 edge
     (255, 120, 192, 1),       # one short of it
@@ -26,10 +30,12 @@ U = 2.0 ** -24
     (1290, 392, 128, 1),      # 11 and 6 M-tiles: last group of four not full
     (33, 40, 704, 1), (31, 24, 768, 1), (65, 72, 832, 1), (63, 56, 896, 1),   # 11 to 14 steps: each tail of the steps in fours
     (65, 72, 640, 1), (63, 56, 576, 1),   # around a 64 edge; 10 and 9 steps (odd and even tails of the step pairs)
-    (300, 520, 1024, 4), (128, 256, 384, 3)])
+    (300, 520, 1024, 4), (128, 256, 384, 3)]
+
+
+@pytest.mark.parametrize('tile,kn,M,N,Kd,split', tiles_for([(kn, *s) for kn in (False, True) for s in TAILS],
+                                                           lambda s: s[0], lambda s: s[4]))
 def test_pipe_tiles_tails(gpu, tile, kn, M, N, Kd, split):
-    if tile == 17 and (kn or split > 1):
-        pytest.skip('tile 17 takes B as [N][K] and no split')
     from chestnut import kernels as K
     print(f'[gemm] pipe tile {tile} kn={kn} {M}x{N}x{Kd} split {split}', flush=True)
     rng = np.random.default_rng(M + N + Kd + tile)
@@ -40,14 +46,12 @@ def test_pipe_tiles_tails(gpu, tile, kn, M, N, Kd, split):
     _gemm_check(C - b, A, B, transB=not kn, depth=Kd // 16 + 40)
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16, 17])
-@pytest.mark.parametrize('kn,N,ldc', [(False, 201, 201), (False, 200, 203), (True, 200, 203)])
-@pytest.mark.parametrize('split', [1, 2])
+@pytest.mark.parametrize('tile,kn,N,ldc,split', tiles_for(
+    [(kn, N, ldc, split) for kn, N, ldc in [(False, 201, 201), (False, 200, 203), (True, 200, 203)] for split in (1, 2)],
+    lambda s: s[0], lambda s: s[3]))
 def test_pipe_tiles_without_16_byte_stores(gpu, tile, kn, N, ldc, split):
     """N odd, or a row pitch that is no multiple of 16 bytes: stored per
     element, and nothing outside [M][N] written."""
-    if tile == 17 and (kn or split > 1):
-        pytest.skip('tile 17 takes B as [N][K] and no split')
     from chestnut import _lib
     torch = gpu
     M, Kd = 150, 256
@@ -65,12 +69,10 @@ def test_pipe_tiles_without_16_byte_stores(gpu, tile, kn, N, ldc, split):
     assert (got[:, N:] == 7.0).all()
 
 
-@pytest.mark.parametrize('tile', [1, 9, 16, 17])
-@pytest.mark.parametrize('M,N,split', [(200, 264, 1), (200, 260, 1), (130, 264, 2)])
+@pytest.mark.parametrize('tile,M,N,split', tiles_for([(200, 264, 1), (200, 260, 1), (130, 264, 2)],
+                                                     lambda s: False, lambda s: s[2]))
 @pytest.mark.parametrize('epi', [1, 2, 3, 4])
 def test_pipe_tiles_epilogues(gpu, tile, M, N, split, epi):
-    if tile == 17 and split > 1:
-        pytest.skip('tile 17 does not split K')
     from chestnut import kernels as K
     torch = gpu
     rng = np.random.default_rng(epi + N)
