@@ -1,6 +1,6 @@
 """BASELINE configs 1-3 as stand-alone workloads for timing and rocprofv3.
 
-    python -m chestnut.configs --config 1|2|3|chain|frames39|stream [--reps N] [--warmup-ms MS] [--out PATH]
+    python -m chestnut.configs --config 1|2|3|kernels|chain|frames39|stream [--reps N] [--warmup-ms MS] [--out PATH]
 
 Each run first copies 256 MiB device to device (the calibration dispatch the
 FETCH_SIZE / WRITE_SIZE summaries scale by), runs the config's kernels
@@ -19,6 +19,12 @@ counter passes.
   3  one pre-LN block of the 1B model (d 2048, 16 x 128 heads, T 512, MLP
      8192), x ~ N(0, 1): the plan entries blkL.ln1 .. blk(L+1).ln1 of a
      4-block engine, each block with its own 100 MB of weights
+  kernels  the per-kernel entry points whose kernels the frame does not use, `reps`
+     launches of each back to back: the pipelined GEMM on 256x128 tiles (4096^3, B as
+     [N][K] and as [K][N]), 128x128 (512 x 8192 x 2048, bias + GELU) and 64x64
+     (1000 x 1000 x 1024), the 32x32 tile (200 x 520 x 2048, residual), row-layout
+     attention (16 heads of 128, 512 tokens); beside them the rate of torch's
+     own 8192^3 f16 product, B as [N][K]
   chain  the cost of a dependent launch (ck_time_launch_chain): chains of
      1000 launches of a near-empty kernel on 1, 256 and 1024 workgroups,
      plain and as one graph; and frame-sized graphs (38 launches, the 39M
@@ -169,6 +175,68 @@ def config3(torch, reps, warmup_ms=0):
         eng.close()
 
 
+def entry_kernels(torch, reps, warmup_ms=0):
+    from . import kernels as K
+    g = torch.Generator(device='cuda').manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, device='cuda', generator=g)  # noqa: E731
+    h = lambda *s: (rnd(*s) / np.sqrt(s[-1])).half()  # noqa: E731
+    n_copies = lambda byts: int(320e6 / byts) + 1  # noqa: E731  (more than the 256 MB Infinity Cache)
+    # name, M, N, K, B as [K][N], epilogue, tile
+    gemms = [('gemm 4096x4096x4096 (tile 9)', 4096, 4096, 4096, False, 0, 9),
+             ('gemm 4096x4096x4096, B [K][N] (tile 9)', 4096, 4096, 4096, True, 0, 9),
+             ('gemm 512x8192x2048 GELU (tile 1)', 512, 8192, 2048, False, 3, 1),
+             ('gemm 1000x1000x1024 (tile 16)', 1000, 1000, 1024, False, 0, 16),
+             ('gemm 200x520x2048 residual (tile 17)', 200, 520, 2048, False, 4, 17)]
+    calls, alg = [], {}
+    for name, M, N, Kd, kn, epi, tile in gemms:
+        plan = K.gemm_workspace(M, N, Kd, kn)
+        if plan[:2] != (tile, 1):
+            raise SystemExit(f'{name}: the planner has tile {plan[0]}, split {plan[1]}')
+        alg[name] = {'flops': 2.0 * M * N * Kd,
+                     'bytes': 2.0 * (M + N) * Kd + 4.0 * N + M * N * {0: 4.0, 3: 2.0, 4: 8.0}[epi]}
+        n = n_copies(alg[name]['bytes'])
+        A = [h(M, Kd) for _ in range(n)]
+        B = [h(Kd, N) if kn else h(N, Kd) for _ in range(n)]
+        b = rnd(N)
+        C = [torch.zeros(M, N, device='cuda', dtype=torch.float16 if epi == 3 else torch.float32) for _ in range(n)]
+        if epi:
+            calls.append(lambda i, n=n, A=A, B=B, C=C, b=b, e=epi: K.gemm_epi(A[i % n], B[i % n], b, e, C[i % n]))
+        else:
+            calls.append(lambda i, n=n, A=A, B=B, C=C, b=b, k=kn: K.gemm(A[i % n], B[i % n], b_kn=k, bias=b, out=C[i % n]))
+    T, H, hd = 512, 16, 128
+    name = 'attention 16 x 128, 512 tokens (row layout)'
+    alg[name] = {'flops': 4.0 * T * T * H * hd, 'bytes': 8.0 * T * H * hd}
+    m = n_copies(alg[name]['bytes'])
+    qk, vt = [rnd(T, 2 * H * hd).half() for _ in range(m)], [rnd(H * hd, T).half() for _ in range(m)]
+    calls.append(lambda i: K.attention(qk[i % m], vt[i % m], H, hd))
+
+    def one_pass():   # all launches of an entry, then the next entry's
+        for c in calls:
+            for i in range(reps):
+                c(i)
+    one_pass()
+    torch.cuda.synchronize()
+    warm(torch, one_pass, warmup_ms)
+    e0, e1 = _events(torch)
+    e0.record()
+    one_pass()
+    e1.record()
+    torch.cuda.synchronize()
+    us = e0.elapsed_time(e1) * 1e3 / reps
+    a, bt = h(8192, 8192), h(8192, 8192).t()
+    warm(torch, lambda: a @ bt, warmup_ms)
+    e0.record()
+    for _ in range(100):
+        a @ bt
+    e1.record()
+    torch.cuda.synchronize()
+    return {'config': 'kernels', 'workload': 'the entry points whose kernels the frame does not use',
+            'unit': 'launch of each', 'sequence': list(alg), 'by_entry': True, 'units_timed': reps, 'us_per_unit': us,
+            'flops': sum(v['flops'] for v in alg.values()), 'bytes': sum(v['bytes'] for v in alg.values()),
+            'bound': 'mfma', 'algorithmic': alg,
+            'torch_8192_product_tflops': 100 * 2.0 * 8192 ** 3 / (e0.elapsed_time(e1) * 1e-3) / 1e12}
+
+
 def launch_chain(torch, reps=0, warmup_ms=0):
     import ctypes
     from ._lib import call
@@ -275,8 +343,8 @@ def frames39(torch, reps=0, warmup_ms=300.0):
 
 def main(argv=None):
     ap = argparse.ArgumentParser(prog='python -m chestnut.configs')
-    ap.add_argument('--config', required=True, choices=('1', '2', '3', 'chain', 'frames39', 'stream'))
-    ap.add_argument('--reps', type=int, default=0, help='timed launches (default: 120 / 200 / 10)')
+    ap.add_argument('--config', required=True, choices=('1', '2', '3', 'kernels', 'chain', 'frames39', 'stream'))
+    ap.add_argument('--reps', type=int, default=0, help='timed launches (default: 120 / 200 / 10, kernels 400)')
     ap.add_argument('--warmup-ms', type=float, default=300.0,
                     help='untimed repetitions for about this much GPU time before the timed ones')
     ap.add_argument('--out', default=None, help='write the run description as JSON')
@@ -290,6 +358,8 @@ def main(argv=None):
         res = launch_chain(torch)
     elif a.config == 'frames39':
         res = frames39(torch, a.reps, a.warmup_ms)
+    elif a.config == 'kernels':
+        res = entry_kernels(torch, a.reps or 400, a.warmup_ms)
     elif a.config == 'stream':
         res = operand_stream(torch, a.reps)
     else:

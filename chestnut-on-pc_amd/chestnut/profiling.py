@@ -282,6 +282,8 @@ def _units(values, run):
     vals = values[-n * len(seq):]
     if len(vals) < n * len(seq):
         raise SystemExit(f'expected {n * len(seq)} dispatches, found {len(vals)}')
+    if run.get('by_entry'):   # all launches of an entry, then the next entry's
+        return {e: vals[k * n:(k + 1) * n] for k, e in enumerate(seq)}
     skip = run.get('blocks_per_rep', 0)
     out = {e: [] for e in seq}
     for u in range(n):
@@ -349,11 +351,13 @@ def configs_md(res, cmd):
     run = res['run']
     alg = run['algorithmic']
     unit_us = sum(e['median_us'] for e in res['entries'].values())
+    units = 'launches of each kernel' if run.get('by_entry') else run['unit'] + 's'
     t_min = max(run['flops'] / (PEAK_TFLOPS * 1e6), run['bytes'] / (PEAK_GBS * 1e3))
-    out = [f"# BASELINE config {run['config']}: {run['workload']}", '',
+    title = run['workload'] if run['config'] == 'kernels' else f"BASELINE config {run['config']}: {run['workload']}"
+    out = [f"# {title[0].upper()}{title[1:]}", '',
            'Commands (run from the repository root on the MI355X box; the counter passes each a run of their own):',
            '', '```', cmd, '```', '',
-           f"Timed: {run['units_timed']} {run['unit']}s over rotating operand copies (more than the 256 MB Infinity "
+           f"Timed: {run['units_timed']} {units} over rotating operand copies (more than the 256 MB Infinity "
            f"Cache), after one untimed pass" + (f" and {run['warmup_ms']:.0f} ms of untimed repetitions (the "
            "GPU's clocks ramp up over the first tens of milliseconds of sustained load)"
            if run.get('warmup_ms') else '') + f".  Kernel trace: {unit_us:.2f} us per {run['unit']} (the sum of the "
@@ -362,6 +366,9 @@ def configs_md(res, cmd):
            f"{t_min:.2f} us, so the {run['unit']} runs at {t_min / unit_us:.3f} of its roofline.  (The HIP-event "
            f"time of the traced run, {run['us_per_unit']:.2f} us per {run['unit']}, includes the tracer's own "
            'per-launch host cost.)', '']
+    if 'torch_8192_product_tflops' in run:
+        out += [f"torch's own 8192x8192x8192 f16 product (B as [N][K]) in the same process: {run['torch_8192_product_tflops']:.0f} "
+                'TFLOP/s.', '']
     if 'split_k' in run:
         out += [f"Planner choice: tile {run['tile']}, split-K {run['split_k']}, workspace {run['workspace_bytes']} B.",
                 '']
