@@ -27,7 +27,8 @@ from . import spec as _spec
 
 FAMILIES = ('qkv', 'o', 'up', 'down')        # per-block GEMMs (every layer gets the choice)
 SINGLE = ('stem0', 'stem1', 'stem2', 'stem3', 'stem4', 'embed')   # once-per-frame GEMMs
-# tile code -> (rows, columns) of the output tile (the codes of ck_gemm)
+# tile code -> (rows, columns) of the output tile (the codes of ck_gemm; its 16 and
+# 17, 64x64 and 32x32 for the row-major outputs, are not tried on frames)
 TILES = {1: (128, 128), 2: (128, 64), 3: (64, 128), 4: (64, 64), 5: (128, 128), 6: (128, 64), 7: (64, 128),
          8: (64, 64), 9: (256, 128), 10: (128, 96), 15: (32, 64)}
 

@@ -1306,13 +1306,23 @@ int auto_split(long tiles, int ksteps) {
 // Where 128x128 tiles number 64 or more: the tile whose estimated time is least
 // of 128x128 (with its automatic split), 256x128 and 64x64.  The estimates (us:
 // a fixed part, a part per 64-wide K-step of a CU's tile, per wave of 256
-// workgroups; two 64x64 workgroups share a CU) are fitted to replayed launches:
-//   128x128:  1000x1000x128 6.6, 128x8192x512 9.7, 1504x1504x1536 16.4,
-//             512x8192x2048 22, 2048x4096x2048 (two waves) 42.4
-//   256x128:  2048x4096x256 13.2, 2048x4096x2048 36.2
-//   64x64:    1000x1000x128 4.4, 128x8192x512 5.4, 1000x1000x1024 8.7 (128x128
-//             split in 4: 19.4), 1504x1504x1536 21.3, 700x3000x256 8.2
-//   reduce:   3 to 4 us and its bytes
+// workgroups; two 64x64 workgroups share a CU; a reduce 3 to 4 us and its bytes)
+// are there to rank the tiles and are not the launch's time: within 10% for one
+// wave of 128x128 or 64x64 workgroups and a short K, 10-30% low for the large
+// tiles otherwise, and up to twice too high for several waves of 64x64.  Replayed
+// launches, us, measured (estimate), f32 out, f16 [N][K] B:
+//                     128x128       256x128       64x64
+//   1000x1000x128       7.1 (6.4)    10.0 (8.1)     4.1 (3.7)
+//   128x8192x512       10.3 (9.2)    14.1 (13.1)    6.2 (5.9)
+//   700x3000x256        8.5 (7.3)    11.8 (9.8)     8.1 (8.7)    the estimate's pick costs 0.4 us
+//   1000x1000x1024     18.9 (15.7)                  9.3 (8.8)    128x128 split in 4
+//   1504x1504x1536     17.0 (16.5)   24.1 (26.2)   19.6 (25.8)
+//   512x8192x2048      23.8 (20.2)   30.4 (32.7)   32.1 (57.2)
+//   2048x4096x256      17.1 (13.2)   13.2 (9.8)    16.7 (33.4)   128x128: two waves
+//   1024x8192x512      22.8 (16.9)   19.8 (13.1)                 two waves
+//   3072x4096x512      31.8 (24.5)   31.1 (24.6)                 three and two waves
+//   2048x4096x2048     45.4 (38.9)   37.1 (32.7)   60.9 (114)    two waves, one
+//   4096x4096x4096    160.8 (135.3) 131.1 (116.5)                four and two waves
 // 64x64 is tile 4 (two K-groups) for a few K-steps and for more of them tile 16
 // (pipelined, as many chains of roundings as the split it replaces).
 int tile_of_many(const GemmDesc& d) {
@@ -1337,8 +1347,12 @@ int tile_of_many(const GemmDesc& d) {
 // the other): 200x520x2048 5.9 / 7.9 (split 4), 16x4096x4096 8.5 / 12.2 (split 4),
 // 11x6272x832 4.7 / 7.3, 600x600x4096 14.1 / 15.8 (split 2), 256x2048x512 5.0 / 4.7,
 // 1x1024x8192 11.7 / 10.0 (split 16); a call of two launches takes 8 us of host
-// time at least.  Not where the split has more chains of roundings than the 16
-// that tile 17 sums an element in.
+// time at least.  Over 153 sizes drawn from 1..4096 x 8..8192 x 64..8192 where it
+// chooses tile 17: 1.38x faster on (geometric) average than tile 4 as it was split,
+// 11 of them slower by more than 2% in graph replays: one K-step (597x432x64 3.7 /
+// 3.2) and a few splits (402x45x7296 13.3 / 12.3 in 6, 6x195x3520 8.6 / 7.7 in 11).
+// Not where the split has more chains of roundings than the 16 that tile 17 sums
+// an element in.
 bool small_tiles_win(const GemmDesc& d) {
   const int ks = d.K / BK;
   const auto tiles = [&](int bm, int bn) { return (long)ceil_div(d.M, bm) * ceil_div(d.N, bn) * d.batch; };
@@ -1364,9 +1378,14 @@ size_t gemm_plan(GemmDesc& d) {
   CK_REQUIRE(d.K % BK == 0, "gemm: K must be a multiple of 64 (pad K)");
   if (d.tile == 0 && d.b_kn && d.split == 0 && d.N % 64 == 0) {
     // A [K][N] B with enough 128x64 tiles to fill the GPU at a split whose K
-    // per split makes whole 3-step phases of the register-staged kernel:
-    // that kernel (config 1: 30.0-31.3 us at split 2, against 31.2-32.6 us
-    // for the 128x128 transposing-read tile at split 4).
+    // per split makes whole 3-step phases of the kernel that brings B in
+    // through registers: that kernel.  Replayed launches, us, against the
+    // pipelined 128x128 and 64x64 tiles: 1024x1024x6144 27.3 at split 2 / 28.1
+    // at split 4 / 37.4; 512x4096x3072 25.5 unsplit / 27.0 at split 2 / 26.8;
+    // 1536x1024x2304 19.4 / 21.4 / 19.8; 1024x2048x1536 16.0 / 18.4 / 15.8.  The
+    // rule does not follow the 64x64 tile where that is ahead (a shorter K, most
+    // of all at split 2): 1024x2048x768 11.1 / 13.2 / 10.4, 512x2048x3072 19.8 /
+    // 22.3 / 17.3, 1024x1024x2304 17.4 / 22.2 / 14.4.
     const long t2 = (long)ceil_div(d.M, 128) * (d.N / 64) * d.batch;
     int s2 = 0;
     for (int c = 1; c <= 8; ++c)

@@ -24,14 +24,28 @@
 // LDS-DMA load in flight has landed (vmcnt(0)), which serialises the ring; the
 // reads of a slice are therefore one asm block that ends with their own wait.
 //
-// Measured on one card, us per call (TFLOP/s), before = the 128x128 tile of
-// gemm.hip with two K-groups:
-//   4096x4096x4096, B [N][K]: 245 (560) -> 126 (1090) on 256x128 (128x128 here 150)
-//   4096x4096x4096, B [K][N]: 245 (560) -> 133 (1030) on 256x128 (128x128 158)
-//   2048x4096x2048, B [N][K]: 59 (580) -> 36 (950) on 256x128 (128x128 42)
-//   2048x4096x2048, B [K][N]: 66 (520) -> 38 (910) on 256x128 (128x128 45)
-//   512x8192x2048,  B [N][K]: 29 (590) -> 22 (775) on 128x128; [K][N] 33 -> 24
-//   1000x2184x1984, B [N][K]: 24.6 (350) -> 18.2 (476) on 128x128; [K][N] 31.3 -> 21.2
+// Measured on one card, graph replays, us per launch (TFLOP/s), before = the
+// 128x128 LDS-DMA tile with two K-groups.  Warm: two sets of operands, in the
+// Infinity Cache where they fit; cold: 700 MB of them in turn.
+//                              before        128x128         256x128
+//   4096x4096x4096 [N][K] warm 246 (558)     156 (880)       132 (1040)
+//                         cold 248 (555)     166 (826)       136 (1008)
+//   4096x4096x4096 [K][N] warm 246 (559)     167 (821)       138 (1000)
+//                         cold 251 (548)     174 (790)       142 (966)
+//   2048x4096x2048 [N][K] warm 58.8 (584)    48.3 (711)      40.2 (855)
+//                         cold 59.0          51.0            40.8
+//   2048x4096x2048 [K][N] warm 66.1 (520)    50.9 (675)      41.4 (830)
+//                         cold 67.9          52.0            41.4
+//   512x8192x2048  [N][K] warm 31.2 (551)    26.1 (658)      29.6
+//                         cold 29.2          27.8            35.2
+//   512x8192x2048  [K][N] warm 34.3 (501)    27.3 (629)      32.6
+//                         cold 32.2          27.4            34.7
+//   1000x2184x1984 [N][K] warm 26.4 (328)    20.3 (427)      29.7
+//                         cold 25.6          24.5            34.0
+//   1000x2184x1984 [K][N] warm 32.3 (268)    22.9 (378)      32.7
+//                         cold 31.3          26.5            37.0
+// (4096x4096x4096, one set of operands for a second: 125 us on normal data, 119 on
+// uniform, 88 on zeros; the power they draw sets the clock.)
 // A 256x256 tile (8 waves, 113 us for 4096x4096x4096) has no registers for the
 // second accumulator of each product that keeps the rounding error at what it was.
 #include <type_traits>
@@ -217,8 +231,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, BM == 64 && S <= 4 ? 2 : 1) void ge
   using I3 = std::integral_constant<int, 3>;
 
   // One k-slice: the MFMAs of the fragments in buffer KK & 1, the reads of the
-  // next slice (slice RK of the stage at `rso`) and NI / 4 refill loads placed
-  // between them.
+  // next slice (slice RK of the stage at `rso`) and the refill loads [DLO, DHI)
+  // of a K-step placed between them.
   auto slice = [&](auto KK, auto RK, bool reads, unsigned rso, bool refill, lwr_t rst, gptr_t ra, gptr_t rb, auto DLO, auto DHI) {
     constexpr int cur = decltype(KK)::value & 1;
     using NX = std::integral_constant<int, 1 - cur>;

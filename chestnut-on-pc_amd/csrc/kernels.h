@@ -38,7 +38,7 @@ enum Epi {
   EPI_EMBED = 8,          // C32 = acc + bias + pos16[m][n] + ctx[n] (the token embedding:
                           // position table and the per-frame context vector folded in)
   EPI_QKV_FRAG = 7,       // f16(acc + bias) of a [T][3d] QKV product, written in the MFMA
-                          // fragment order the attention kernel loads (see gemm.hip):
+                          // fragment order the attention kernel loads (see gemm_common.h):
                           // Q, K -> C, V -> vt.  Needs head_dim, M % 32 == 0, split 1.
 };
 
@@ -70,7 +70,8 @@ struct GemmDesc {
   half_t* vt = nullptr;        // EPI_QKV transposed V output
   int qk_cols = 0;
   long vt_ld = 0;
-  int tile = 0;                // 0 auto; else 1:128x128 2:128x64 3:64x128 4:64x64
+  int tile = 0;                // 0 auto, else a code of 1..17: see launch_epi (gemm.hip) for the list and
+                               // gemm_plan for the epilogues and layouts each takes
   int head_dim = 0;            // EPI_QKV_FRAG only
   const half_t* pos = nullptr; // EPI_EMBED: f16 [M][N] position table (row stride ldc)
   const float* ctx = nullptr;  // EPI_EMBED: f32 [N] added to every row
